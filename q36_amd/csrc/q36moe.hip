@@ -1391,9 +1391,9 @@ __global__ __launch_bounds__(256, 2) void k_gateup_dma(GemmArgs A) {
 // logits[t][r] = W[r] . x[t] for r < n_expert; row n_expert (when present)
 // is the shared-expert gate, written to shg[t].  Two numerics, as the
 // reference has two paths:
-//   k_router_f32: fp32 products and sums, one wavefront per row (decode:
+//   k_router_f32: fp32 products and sums, one wavefront per row and token (decode:
 //     k_matvec_f32_row, q36_ops.cuh:331-342); the row stays in registers
-//     while every token's dot product is formed.
+//     while its tokens' dot products are formed.
 //   k_router_f16: W and x rounded to fp16 (RNE), fp32 accumulation on
 //     v_mfma_f32_16x16x32_f16 (prefill: pf_gemm's fp16 tensor-core path,
 //     q36_engine.cu:3403-3414, 2365-2384).
@@ -1405,100 +1405,266 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(64) void k_router_f32(const float *__restrict__ W, int n_expert,
-                                                   const void *__restrict__ x, int x_fmt, int T,
-                                                   float *__restrict__ logits, int ld,
-                                                   float *__restrict__ shg) {
-    const int r = blockIdx.x, lane = threadIdx.x;
+// Workgroup = one router row, wave w = NT tokens (w, w + waves, ...): the
+// tokens' dot products run side by side, where one wave walking the tokens
+// paid an L2 round trip for each.  At most kRfW waves, so that a wave's row
+// and tokens are all in flight at once (16 waves leave 64 registers each,
+// which a row and a token fill).  Same products and order of sums whatever T.
+// us at T = 1 / 4 / 7 / 16, 257 rows: 2.4 / 3.6 / 4.9 / 8.7 with one wave per
+// row walking the tokens, 2.5 / 2.8 / 3.4 / 4.9 now (1: a launch's floor).
+constexpr int kRfW = 8;
+template <int XF, int NT>
+__global__ __launch_bounds__(64 * kRfW) void k_router_f32(const float *__restrict__ W, int n_expert,
+                                                         const void *__restrict__ x, int T,
+                                                         float *__restrict__ logits, int ld,
+                                                         float *__restrict__ shg) {
+    const int r = blockIdx.x, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const float *w = W + (size_t)r * kRtD;
     float4 wv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) wv[j] = *reinterpret_cast<const float4 *>(w + (j * 64 + lane) * 4);
-    for (int t = 0; t < T; t++) {
-        float xv[32];
-        if (x_fmt == Q36MOE_FMT_F32) {
-            const float *xt = static_cast<const float *>(x) + (size_t)t * kRtD;
+    for (int t0 = wave; t0 < T; t0 += nw * NT) {
+        u32x4 xf[NT][8];   // fp32 x
+        uint2 xh[NT][8];   // bf16 x
+#pragma unroll
+        for (int u = 0; u < NT; u++) {
+            const size_t o = (size_t)min(t0 + u * nw, T - 1) * kRtD;   // past the end: the last token again, not stored
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const float4 v = *reinterpret_cast<const float4 *>(xt + (j * 64 + lane) * 4);
-                xv[4 * j] = v.x; xv[4 * j + 1] = v.y; xv[4 * j + 2] = v.z; xv[4 * j + 3] = v.w;
+                if constexpr (XF == Q36MOE_FMT_F32)
+                    xf[u][j] = *reinterpret_cast<const u32x4 *>(static_cast<const float *>(x) + o + (j * 64 + lane) * 4);
+                else
+                    xh[u][j] = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(x) + o + (j * 64 + lane) * 4);
             }
-        } else {
-            const uint16_t *xt = static_cast<const uint16_t *>(x) + (size_t)t * kRtD;
+        }
+        // every load issued before the first product: left alone, the compiler
+        // keeps four of a token's eight in flight
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < NT; u++) {
+            float acc = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const uint2 v = *reinterpret_cast<const uint2 *>(xt + (j * 64 + lane) * 4);
-                xv[4 * j] = __uint_as_float(v.x << 16); xv[4 * j + 1] = __uint_as_float(v.x & 0xffff0000u);
-                xv[4 * j + 2] = __uint_as_float(v.y << 16); xv[4 * j + 3] = __uint_as_float(v.y & 0xffff0000u);
-            }
-        }
-        float acc = 0.0f;
+                float xv[4];
+                if constexpr (XF == Q36MOE_FMT_F32) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            acc = fmaf(wv[j].x, xv[4 * j], acc);
-            acc = fmaf(wv[j].y, xv[4 * j + 1], acc);
-            acc = fmaf(wv[j].z, xv[4 * j + 2], acc);
-            acc = fmaf(wv[j].w, xv[4 * j + 3], acc);
-        }
-        acc = wave_sum(acc);
-        if (lane == 0) {
-            if (r < n_expert) logits[(size_t)t * ld + r] = acc;
-            else shg[t] = acc;
+                    for (int i = 0; i < 4; i++) xv[i] = __uint_as_float(xf[u][j][i]);
+                } else {
+                    xv[0] = __uint_as_float(xh[u][j].x << 16); xv[1] = __uint_as_float(xh[u][j].x & 0xffff0000u);
+                    xv[2] = __uint_as_float(xh[u][j].y << 16); xv[3] = __uint_as_float(xh[u][j].y & 0xffff0000u);
+                }
+                acc = fmaf(wv[j].x, xv[0], acc);
+                acc = fmaf(wv[j].y, xv[1], acc);
+                acc = fmaf(wv[j].z, xv[2], acc);
+                acc = fmaf(wv[j].w, xv[3], acc);
+            }
+            acc = wave_sum(acc);
+            const int t = t0 + u * nw;
+            if (lane == 0 && t < T) {
+                if (r < n_expert) logits[(size_t)t * ld + r] = acc;
+                else shg[t] = acc;
+            }
         }
     }
 }
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// 8 consecutive activations of token row `t` from K offset k, rounded to fp16
-__device__ __forceinline__ f16x8 x8_f16(const void *x, int x_fmt, size_t off) {
-    float v[8];
-    load8(x, x_fmt, off, v);
-    f16x8 h;
-#pragma unroll
-    for (int i = 0; i < 8; i++) h[i] = (_Float16)v[i];
-    return h;
+// Workgroup = TT token tiles x RT row tiles of 16 (the last row block of a
+// grid of RT = 4 takes a fifth tile when at most 16 rows are left over: 257
+// rows are four blocks, not five), kRhW waves that split K: wave w forms the
+// whole tile's partial sums over K 256w .. 256w+255, so every byte of x and W
+// enters the CU once, and the waves meet only at the end (partial sums
+// through LDS, added in wave order).  A K-step of 32 is loaded with 8 lanes
+// per 128-byte row segment (a load whose neighbouring lanes lie in different
+// rows, as the MFMA operands do, costs the address unit a cycle per lane),
+// rounded to fp16 and passed through the wave's own LDS into operand order;
+// no barrier in the K loop.  NB step buffers: step s + NB is loaded as soon
+// as step s is converted.
+//   v_mfma_f32_16x16x32_f16: lane L holds row (A) or column (B) L%16 and K
+// elements 8(L/16)..8(L/16)+7.
+constexpr int kRhW = 8;
+
+// Byte offset of (row r, K element 4c) in a staged fp16 tile of 16 rows x 64 B:
+// 16-byte slots XORed with the row's high bits, so the 16 rows of a fragment
+// read fall in 16 distinct bank groups.
+__device__ __forceinline__ int rh_off(int r, int c) {
+    return r * 64 + ((((c >> 1) ^ (r >> 2)) & 3) << 4) + ((c & 1) << 3);
 }
 
-// workgroup = 64 router rows x 64 tokens; wave w owns tokens 16w..16w+15
-// and all 4 row tiles.  v_mfma_f32_16x16x32_f16 operands: lane L holds row
-// (A) or column (B) L%16 and K elements 8(L/16)..8(L/16)+7.
-__global__ __launch_bounds__(256) void k_router_f16(const float *__restrict__ W, int n_rows, int n_expert,
-                                                    const void *__restrict__ x, int x_fmt, int T,
-                                                    float *__restrict__ logits, int ld,
-                                                    float *__restrict__ shg) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
-    const int r0 = blockIdx.x * 64, t0 = blockIdx.y * 64 + wave * 16;
-    const int tok = min(t0 + n, T - 1);                  // padding columns repeat the last token
-    int rows[4];
+__device__ __forceinline__ uint32_t f16x2(float a, float b) {
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) |
+           ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
+}
+
+template <int XF, int TT, int RT, int NB>
+__device__ __forceinline__ void router_f16_tile(const float *__restrict__ W, int n_rows, int n_expert,
+                                                const void *__restrict__ x, int T, int t0, int r0,
+                                                float *__restrict__ logits, int ld, float *__restrict__ shg,
+                                                uint8_t *stage, float (*red)[TT * 256]) {
+    constexpr int NS = kRtD / kRhW / 32;   // K-steps per wave
+    constexpr bool F32 = XF == Q36MOE_FMT_F32;
+    constexpr int XB = F32 ? 4 : 2, XI = F32 ? 2 * TT : TT;   // bytes per x value, loads per step
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k0 = wave * (kRtD / kRhW);
+    uint8_t *sx = stage + wave * (TT + RT) * 1024, *sw = sx + TT * 1024;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(static_cast<const uint8_t *>(x) + ((size_t)t0 * kRtD + k0) * XB), (short)0, 0x7ffffffe, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(W + (size_t)r0 * kRtD + k0), (short)0, 0x7ffffffe, 0x00020000);
+    // rows past the end repeat the last one; their results are never stored
+    uint32_t xo[XI], wo[2 * RT];
 #pragma unroll
-    for (int i = 0; i < 4; i++) rows[i] = min(r0 + 16 * i + n, n_rows - 1);
-    v4f acc[4];
+    for (int i = 0; i < XI; i++) {
+        const int r = F32 ? 8 * i + (lane >> 3) : 16 * i + (lane >> 2);
+        xo[i] = (uint32_t)min(r, T - 1 - t0) * (kRtD * XB) + (F32 ? lane & 7 : lane & 3) * 16;
+    }
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < kRtD; k0 += 32) {
-        const f16x8 b = x8_f16(x, x_fmt, (size_t)tok * kRtD + k0 + 8 * g);
+    for (int i = 0; i < 2 * RT; i++)
+        wo[i] = (uint32_t)min(8 * i + (lane >> 3), n_rows - 1 - r0) * (kRtD * 4) + (lane & 7) * 16;
+    v4f acc[RT][TT];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float *wr = W + (size_t)rows[i] * kRtD + k0 + 8 * g;
-            const float4 w0 = *reinterpret_cast<const float4 *>(wr);
-            const float4 w1 = *reinterpret_cast<const float4 *>(wr + 4);
-            const f16x8 a = f16x8{(_Float16)w0.x, (_Float16)w0.y, (_Float16)w0.z, (_Float16)w0.w,
-                                  (_Float16)w1.x, (_Float16)w1.y, (_Float16)w1.z, (_Float16)w1.w};
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[i], 0, 0, 0);
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int j = 0; j < TT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    struct Step { u32x4 xv[XI], wv[2 * RT]; } st[NB];
+    auto load = [&](int s, Step &o) {
+#pragma unroll
+        for (int i = 0; i < XI; i++) o.xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i], s * 32 * XB, 0);
+#pragma unroll
+        for (int i = 0; i < 2 * RT; i++) o.wv[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo[i], s * 128, 0);
+    };
+    auto put4 = [&](uint8_t *tile, int r, const u32x4 &v) {   // 4 fp32 -> 8 bytes
+        const int o = (r >> 4) * 1024 + rh_off(r & 15, lane & 7);
+        *reinterpret_cast<uint2 *>(tile + o) = make_uint2(f16x2(__uint_as_float(v[0]), __uint_as_float(v[1])),
+                                                         f16x2(__uint_as_float(v[2]), __uint_as_float(v[3])));
+    };
+#pragma unroll
+    for (int s = 0; s < NB; s++) load(s, st[s]);
+    static_assert(NS % NB == 0, "whole groups of NB steps");
+    auto group = [&](int s0, auto LASTC) {
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            Step &c = st[u];
+#pragma unroll
+            for (int i = 0; i < XI; i++) {
+                if constexpr (F32) {
+                    put4(sx, 8 * i + (lane >> 3), c.xv[i]);
+                } else {   // 8 bf16 -> 16 bytes
+                    u32x4 h;
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        h[v] = f16x2(__uint_as_float(c.xv[i][v] << 16), __uint_as_float(c.xv[i][v] & 0xffff0000u));
+                    *reinterpret_cast<u32x4 *>(sx + i * 1024 + rh_off(lane >> 2, 2 * (lane & 3))) = h;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2 * RT; i++) put4(sw, 8 * i + (lane >> 3), c.wv[i]);
+            if constexpr (!decltype(LASTC)::value) load(s0 + u + NB, c);
+            route_sync();   // the wave's writes before its reads
+            f16x8 b[TT];
+#pragma unroll
+            for (int j = 0; j < TT; j++) b[j] = *reinterpret_cast<const f16x8 *>(sx + j * 1024 + rh_off(n, 2 * g));
+#pragma unroll
+            for (int i = 0; i < RT; i++) {
+                const f16x8 a = *reinterpret_cast<const f16x8 *>(sw + i * 1024 + rh_off(n, 2 * g));
+#pragma unroll
+                for (int j = 0; j < TT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[j], acc[i][j], 0, 0, 0);
+            }
+            route_sync();   // and its reads before the next step's writes
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll 1
+    for (int s0 = 0; s0 < NS - NB; s0 += NB) group(s0, std::false_type{});
+    group(NS - NB, std::true_type{});
+    // C: lane L holds rows 4(L/16)+c of token column L%16; red[wave] is
+    // [token of the tile][16 rows]
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+        if (i > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < TT; j++) *reinterpret_cast<v4f *>(&red[wave][(16 * j + n) * 16 + 4 * g]) = acc[i][j];
+        __syncthreads();
+        for (int o = tid; o < TT * 256; o += 64 * kRhW) {
+            float v = red[0][o];
+#pragma unroll
+            for (int w = 1; w < kRhW; w++) v += red[w][o];
+            const int t = t0 + (o >> 4), r = r0 + 16 * i + (o & 15);
+            if (t < T) {
+                if (r < n_expert) logits[(size_t)t * ld + r] = v;
+                else if (r < n_rows) shg[t] = v;
+            }
         }
     }
-    // C: lane L holds rows 4(L/16)+j of token column L%16
-    const int t = t0 + n;
-    if (t >= T) return;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = r0 + 16 * i + 4 * g + j;
-            if (r < n_expert) logits[(size_t)t * ld + r] = acc[i][j];
-            else if (r < n_rows) shg[t] = acc[i][j];
+}
+
+template <int XF, int TT, int RT, int NB>
+__global__ __launch_bounds__(64 * kRhW) void k_router_f16(const float *__restrict__ W, int n_rows, int n_expert,
+                                                          const void *__restrict__ x, int T, int nrb,
+                                                          float *__restrict__ logits, int ld,
+                                                          float *__restrict__ shg) {
+    constexpr int RX = RT == 4 ? 5 : RT;
+    __shared__ __align__(16) uint8_t stage[kRhW * (TT + RX) * 1024];
+    __shared__ __align__(16) float red[kRhW][TT * 256];
+    // the row blocks of one token block run back to back on one XCD, whose L2
+    // then holds its x
+    const int xcd = blockIdx.x & 7, jx = blockIdx.x >> 3;
+    const int t0 = (8 * (jx / nrb) + xcd) * 16 * TT, rb = jx % nrb;
+    if (t0 >= T) return;
+    if constexpr (RT == 4) {
+        if (rb == nrb - 1 && n_rows - rb * 64 > 64) {
+            router_f16_tile<XF, TT, 5, NB>(W, n_rows, n_expert, x, T, t0, rb * 64, logits, ld, shg, stage, red);
+            return;
         }
+    }
+    router_f16_tile<XF, TT, RT, NB>(W, n_rows, n_expert, x, T, t0, rb * 16 * RT, logits, ld, shg, stage, red);
+}
+
+// A workgroup's time is that of bringing its tile's rows in through one CU
+// (8 KiB per router row and fp32 token), so small tiles win while they leave
+// at most about one and a half workgroups per CU, and large ones, which read
+// x and W fewer times, beyond.  Measured with 257 rows, us per tile shape
+// (token tiles x row tiles), fp32 x:
+//   T        17   203   300   400   700  1000  1400  2000  2800  4096
+//   1 x 1   4.5   6.8   7.1   8.9  11.4  13.8  17.0  23.9  31.9  45.8
+//   2 x 2   6.7   7.6   7.6   7.8   8.1  11.9  12.6  17.0  22.1  29.1
+//   2 x 4  11.1  11.8  11.8  12.1  12.1  12.4  12.9  13.9  23.9  28.5
+//   4 x 4  13.4  15.1  15.5  15.5  15.7  16.0  16.4  17.0  18.0  21.2
+// (one wave per 16 tokens and 64 rows, walking all of K with the operands
+// loaded in MFMA order: 63 at T = 17, 72 at 64 to 2800, 144 at 4096.)
+template <int XF, int TT, int RT, int NB>
+static void launch_router_f16(const float *w, int n_rows, int n_expert, const void *x, int T, int nrb, float *logits,
+                              int ld, float *shg, hipStream_t s) {
+    const unsigned ntb = (unsigned)((T + 16 * TT - 1) / (16 * TT));
+    hipLaunchKernelGGL((k_router_f16<XF, TT, RT, NB>), dim3((ntb + 7) / 8 * 8 * nrb), dim3(64 * kRhW), 0, s, w, n_rows,
+                       n_expert, x, T, nrb, logits, ld, shg);
+}
+
+template <int XF>
+static void launch_router(bool f16, const float *w, int n_rows, int n_expert, const void *x, int T, float *logits,
+                          int ld, float *shg, hipStream_t s) {
+    if (!f16) {
+        if (T <= kRfW)
+            hipLaunchKernelGGL((k_router_f32<XF, 1>), dim3(n_rows), dim3(64 * T), 0, s, w, n_expert, x, T, logits, ld, shg);
+        else
+            hipLaunchKernelGGL((k_router_f32<XF, 2>), dim3(n_rows), dim3(64 * kRfW), 0, s, w, n_expert, x, T, logits, ld, shg);
+        return;
+    }
+    const int nrb1 = (n_rows + 15) / 16, nrb2 = (n_rows + 31) / 32;
+    const int nrb4 = n_rows <= 64 ? 1 : (n_rows - 17) / 64 + 1;   // up to 16 rows left over join the last block
+    auto wgs = [T](int tt, int nrb) { return (long)((T + 16 * tt - 1) / (16 * tt)) * nrb; };
+    if (wgs(1, nrb1) <= 384)
+        launch_router_f16<XF, 1, 1, 4>(w, n_rows, n_expert, x, T, nrb1, logits, ld, shg, s);
+    else if (wgs(2, nrb2) <= 448)
+        launch_router_f16<XF, 2, 2, 2>(w, n_rows, n_expert, x, T, nrb2, logits, ld, shg, s);
+    else if (wgs(2, nrb4) <= 256)
+        launch_router_f16<XF, 2, 4, 2>(w, n_rows, n_expert, x, T, nrb4, logits, ld, shg, s);
+    else
+        launch_router_f16<XF, 4, 4, 1>(w, n_rows, n_expert, x, T, nrb4, logits, ld, shg, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -3604,12 +3770,8 @@ int q36moe_router_logits(const float *w, int n_rows, int n_expert, const void *x
     if (!w || !x || !logits || (n_rows > n_expert && !shg)) return Q36MOE_EINVAL;
     const bool f16 = mode == 2 || (mode == 0 && T > kDirectMaxT);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (f16)
-        hipLaunchKernelGGL(k_router_f16, dim3((n_rows + 63) / 64, (T + 63) / 64), dim3(256), 0, s, w, n_rows,
-                           n_expert, x, x_fmt, T, logits, ld, shg);
-    else
-        hipLaunchKernelGGL(k_router_f32, dim3(n_rows), dim3(64), 0, s, w, n_expert, x, x_fmt, T, logits, ld,
-                           shg);
+    if (x_fmt == Q36MOE_FMT_F32) launch_router<Q36MOE_FMT_F32>(f16, w, n_rows, n_expert, x, T, logits, ld, shg, s);
+    else launch_router<Q36MOE_FMT_BF16>(f16, w, n_rows, n_expert, x, T, logits, ld, shg, s);
     return hip_rc(hipGetLastError());
 }
 

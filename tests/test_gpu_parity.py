@@ -798,6 +798,51 @@ def test_router_logits_bf16_input_and_no_shared(dev):
     assert (np.abs(lg.cpu().numpy() - ref) / mag).max() <= 2e-6
 
 
+# every tile shape of the fp16 router at its edges: 257 rows (the last row
+# block takes a fifth tile) and row counts around a block, T at both sides of
+# each rule and with remainders
+@pytest.mark.parametrize("T,n_expert,n_rows,bf16", [
+    (17, 256, 257, False), (17, 256, 257, True), (337, 256, 257, False), (361, 256, 257, True),
+    (1567, 256, 257, False), (1601, 256, 257, True), (2048, 256, 257, False), (2049, 256, 257, True),
+    (2113, 256, 256, False), (4097, 80, 81, False), (4099, 80, 80, True), (9001, 1, 2, False), (70, 63, 64, False),
+    (12001, 16, 17, True)])
+def test_router_f16_tiles(dev, T, n_expert, n_rows, bf16):
+    rng = np.random.default_rng(700 + T)
+    w = (rng.standard_normal((n_rows, 2048)) * 0.02).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((T, 2048), dtype=np.float32)).to(dev)
+    if bf16:
+        x = x.to(torch.bfloat16)
+    ld = n_expert + 3                       # rows wider than the experts: the rest stays as it was
+    wt = torch.from_numpy(w).to(dev)
+    lg = torch.full((T, ld), 7.0, device=dev)
+    shg = torch.full((T,), 7.0, device=dev)
+    moe.check(moe.lib().q36moe_router_logits(
+        wt.data_ptr(), n_rows, n_expert, x.data_ptr(), 1 if bf16 else 0, T, 2048, 2, lg.data_ptr(), ld,
+        shg.data_ptr() if n_rows > n_expert else None, moe._stream()), "q36moe_router_logits")
+    torch.cuda.synchronize()
+    assert (lg[:, n_expert:] == 7.0).all() and (n_rows > n_expert or (shg == 7.0).all())
+    ref, mag = _router_ref(w, x.float().cpu().numpy(), True)
+    got = torch.cat([lg[:, :n_expert], shg[:, None]], 1)[:, :n_rows].cpu().numpy().astype(np.float64)
+    # fp32 sums of 2048 products in 8 partial sums: well inside 2e-6 of the
+    # sum of the terms' magnitudes, the bar of test_router_logits
+    assert (np.abs(got - ref) / mag).max() <= 2e-6
+
+
+@pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 35])
+def test_router_f32_waves(dev, T):
+    """One wave per token up to 16, a loop beyond: the same sums either way."""
+    rng = np.random.default_rng(800 + T)
+    w = torch.from_numpy((rng.standard_normal((257, 2048)) * 0.02).astype(np.float32)).to(dev)
+    x = torch.from_numpy(rng.standard_normal((T, 2048), dtype=np.float32)).to(dev)
+    lg, shg = moe.router_logits(w, x, 256, moe.ROUTER_F32)
+    one = [moe.router_logits(w, x[t:t + 1].contiguous(), 256, moe.ROUTER_F32) for t in range(T)]
+    torch.cuda.synchronize()
+    assert torch.equal(lg, torch.cat([o[0] for o in one])) and torch.equal(shg, torch.cat([o[1] for o in one]))
+    ref, mag = _router_ref(w.cpu().numpy(), x.cpu().numpy(), False)
+    got = torch.cat([lg, shg[:, None]], 1).cpu().numpy().astype(np.float64)
+    assert (np.abs(got - ref) / mag).max() <= 2e-6
+
+
 @pytest.mark.parametrize("T,with_a", [(1, True), (5, True), (300, True), (7, False)])
 def test_add_rmsnorm_quant(dev, oracle, T, with_a):
     """Fused residual add + RMSNorm + quantisation: h += a bit-exact (one
