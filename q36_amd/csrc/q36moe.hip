@@ -520,7 +520,7 @@ struct RouteArgs {
     const float *logits; int ld; int T; int E; int k; float scale;
     const void *x; int x_fmt; int D; int nb;
     int32_t *idx; float *wt; uint8_t *xq; uint8_t *xs; uint8_t *xs2;
-    int32_t *blk_cnt; int32_t *rank;
+    uint8_t *blk_cnt; int32_t *rank;
     const uint8_t *xs_in;     // scales of pre-quantised x (x_fmt kFmtE4M3)
     int8_t *xq8; float *xsf;  // int8 x + fp32 scales per 32 for a q8_0-split shared expert, or null
     int counts;               // write blk_cnt / rank (0: the one-kernel skinny path sorts itself)
@@ -528,8 +528,8 @@ struct RouteArgs {
 
 // One wavefront per token, TPB tokens per workgroup: top-k routing,
 // FP8 quantisation of x (8 values per lane, 4 lanes per 32-block), then the
-// block's per-expert counts (expert-major, blk_cnt[e][block]) and each
-// entry's rank among the block's earlier entries of the same expert (the
+// block's per-expert counts (one byte each, blk_cnt[block][kMaxExperts]) and
+// each entry's rank among the block's earlier entries of the same expert (the
 // stable order of the sort), from a per-expert mask of the block's tokens.
 // Small batches use 4 tokens per workgroup to spread the quantisation over
 // more CUs; large ones 16, which keeps the per-block count table short.
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(64 * TPB) void k_route(RouteArgs A) {
     const int t0 = blockIdx.x * TPB;
     const int nb32 = A.D / 32;
     if (A.counts) {   // uniform
-        for (int e = threadIdx.x; e < A.E; e += 64 * TPB) tmask[e] = 0u;
+        for (int e = threadIdx.x; e < kMaxExperts; e += 64 * TPB) tmask[e] = 0u;
         __syncthreads();
     }
     const int t = t0 + wave;
@@ -615,8 +615,12 @@ __global__ __launch_bounds__(64 * TPB) void k_route(RouteArgs A) {
         const int e = ent[threadIdx.x];
         A.rank[(size_t)t0 * A.k + threadIdx.x] = __popc(tmask[e] & ((1u << tl) - 1u));
     }
-    for (int e = threadIdx.x; e < A.E; e += 64 * TPB)
-        A.blk_cnt[(size_t)e * A.nb + blockIdx.x] = __popc(tmask[e]);
+    if (threadIdx.x < kMaxExperts / 4) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) c |= (uint32_t)__popc(tmask[4 * threadIdx.x + j]) << (8 * j);
+        reinterpret_cast<uint32_t *>(A.blk_cnt + (size_t)blockIdx.x * kMaxExperts)[threadIdx.x] = c;
+    }
 }
 
 // k_route without the per-block counts (the one-kernel skinny path sorts
@@ -706,7 +710,7 @@ __global__ __launch_bounds__(256) void k_quant(const void *x, int x_fmt, int T, 
 // sort: offsets, stable scatter, tile list
 // ---------------------------------------------------------------------------
 struct ScanArgs {
-    const int32_t *blk_cnt; int nb; int tpb; int inline_cols; int E; int T; int k;
+    const uint8_t *blk_cnt; int nb; int tpb; int inline_cols; int E; int T; int k;
     const int32_t *idx; const float *wt; const int32_t *rank; const float *shg; int ld_shg;
     int tn;      // rows per routed tile
     int tn_sh;   // rows per shared-expert tile
@@ -714,59 +718,59 @@ struct ScanArgs {
     int32_t *row_tok; float *row_w; int4 *tiles; int32_t *ntiles;
 };
 
-// Column scans: for each expert, the exclusive prefix of its per-block counts
-// (blk_off[e][b]) and its total.  kColExp experts per workgroup, 256 / kColExp
-// threads per expert, each summing a contiguous run of blocks.
-constexpr int kColExp = 8;
-constexpr int kScanInlineBlocks = 64;   // k_scatter does the column scan itself up to this many blocks
+// Column scans (past kScanInlineBlocks blocks): for each expert, the exclusive
+// prefix of its per-block counts (blk_off[e][b]) and its total.  kColExp
+// experts per workgroup (one dword of each block's counts), each thread a
+// contiguous run of blocks.
+constexpr int kColExp = 4;
+constexpr int kScanInlineBlocks = 512;   // k_scatter does the column scan itself up to this many blocks
 __global__ __launch_bounds__(256) void k_colscan(ScanArgs A) {
-    constexpr int NP = 256 / kColExp;              // partitions per expert: one half-wave
-    static_assert(NP == 32, "one expert per half-wave");
-    constexpr int CH = 8;                          // counts held in registers per thread
-    const int lane = threadIdx.x & 63;
-    const int el = threadIdx.x / NP, pi = threadIdx.x % NP;
-    const int e = blockIdx.x * kColExp + el;
-    const bool ok = e < A.E;
-    const int chunk = (A.nb + NP - 1) / NP;
-    const int b0 = pi * chunk, b1 = min(A.nb, b0 + chunk);
-    const int32_t *cnt = A.blk_cnt + (size_t)e * A.nb;
-    // all of a thread's counts are loaded at once (one memory round trip)
-    int v[CH], sum = 0;
-    if (chunk <= CH) {
+    __shared__ int wsum[4][kColExp];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int e0 = blockIdx.x * kColExp;
+    const int chunk = (A.nb + 255) / 256;
+    const int b0 = min(A.nb, tid * chunk), b1 = min(A.nb, b0 + chunk);
+    const uint32_t *cnt = reinterpret_cast<const uint32_t *>(A.blk_cnt + e0);
+    constexpr int RS = kMaxExperts / 4;            // dwords of one block's counts
+    int sum[kColExp] = {0, 0, 0, 0};
+    for (int b = b0; b < b1; b++) {
+        const uint32_t c = cnt[(size_t)b * RS];
 #pragma unroll
-        for (int j = 0; j < CH; j++) {
-            v[j] = ok && b0 + j < b1 ? cnt[b0 + j] : 0;
-            sum += v[j];
-        }
-    } else if (ok) {
-        for (int b = b0; b < b1; b++) sum += cnt[b];
+        for (int j = 0; j < kColExp; j++) sum[j] += (c >> (8 * j)) & 255u;
     }
-    // inclusive scan over the expert's 32 lanes: row_shr 1/2/4/8 inside each
-    // 16-lane row, then row_bcast15 adds row 0's (row 2's) total to row 1 (3)
-    int inc = sum;
-    inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
-    inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
-    inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
-    inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
-    inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
-    const int total = __shfl(inc, (lane & 32) | 31, 64);
-    if (!ok) return;
-    int run = inc - sum;
-    if (chunk <= CH) {
+    int run[kColExp];
 #pragma unroll
-        for (int j = 0; j < CH; j++)
-            if (b0 + j < b1) {
-                A.blk_off[(size_t)e * A.nb + b0 + j] = run;
-                run += v[j];
-            }
-    } else {
-        for (int b = b0; b < b1; b++) {
-            const int c = cnt[b];
-            A.blk_off[(size_t)e * A.nb + b] = run;
-            run += c;
+    for (int j = 0; j < kColExp; j++) {
+        // inclusive scan over the wave: row_shr 1/2/4/8, row_bcast15, row_bcast31
+        int inc = sum[j];
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
+        inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
+        run[j] = inc - sum[j];
+        if (lane == 63) wsum[wv][j] = inc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kColExp; j++) {
+        int total = 0;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            run[j] += w < wv ? wsum[w][j] : 0;
+            total += wsum[w][j];
+        }
+        if (tid == 0 && e0 + j < A.E) A.tot[e0 + j] = total;
+    }
+    for (int b = b0; b < b1; b++) {
+        const uint32_t c = cnt[(size_t)b * RS];
+#pragma unroll
+        for (int j = 0; j < kColExp; j++) {
+            if (e0 + j < A.E) A.blk_off[(size_t)(e0 + j) * A.nb + b] = run[j];
+            run[j] += (c >> (8 * j)) & 255u;
         }
     }
-    if (pi == 0) A.tot[e] = total;
 }
 
 // Exclusive scan of v[0..n) (n <= 256) by one wavefront into out (LDS).
@@ -803,12 +807,68 @@ __device__ __forceinline__ void wave_scan256(const int *v, int n, int *out, int 
 // deterministic replacement of the reference's atomic bucketing
 // (k_moe_dispatch, q36_engine.cu:3387-3392): entry ids t*k+s ascend inside
 // each expert.
-// With few routing blocks (inline_cols) each workgroup also does the column
-// scan itself -- every expert's counts over all blocks, a few KiB -- and
-// k_colscan is not launched.
+// Up to kScanInlineBlocks routing blocks (8192 tokens) each workgroup also
+// does the column scan itself (inline_cols) and k_colscan is not launched:
+// the counts are a byte each, 256 per block, so one 16-byte load per lane
+// covers 16 blocks over the workgroup, and all of a lane's loads are in
+// flight together.  A count is at most 16, so the sums over up to 512 blocks
+// fit the bytes' 16-bit widenings.  Beyond, the workgroups' reads grow with
+// the square of the tokens, and the separate scan, which reads each count
+// once, takes over.  us of the scan stage, against a count per int in
+// expert-major order, scanned by each workgroup up to 64 blocks and by
+// k_colscan above:
+//   T = 1000     17.0 -> 5.8            T = 4096   5.1 + 6.0 -> 7.9
+//   T = 8000     8.9 + 7.6 -> 11.0      T = 33000  33 + 12.8 -> 10.0 + 13.6
+constexpr int kScSub = 16;                       // blocks per load round
+template <int R>   // rounds in flight
+__device__ __forceinline__ void scan_block_counts(const uint8_t *cnt, int nb, int b,
+                                                  uint32_t (*part)[2][kMaxExperts / 2], int &tot, int &before) {
+    const int tid = threadIdx.x, sub = tid >> 4, c = tid & 15;
+    uint32_t t[8], f[8];   // experts 16c + 4j + {0, 2} and {1, 3}, 16 bits each: all blocks / those before b
+#pragma unroll
+    for (int j = 0; j < 8; j++) t[j] = f[j] = 0u;
+    for (int r0 = 0; r0 * kScSub < nb; r0 += R) {
+        u32x4 v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int bb = (r0 + r) * kScSub + sub;
+            v[r] = *reinterpret_cast<const u32x4 *>(cnt + (size_t)min(bb, nb - 1) * kMaxExperts + 16 * c);
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int bb = (r0 + r) * kScSub + sub;
+            const uint32_t all = bb < nb ? 0x00ff00ffu : 0u, bef = bb < b ? 0x00ff00ffu : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                t[2 * j] += v[r][j] & all;
+                t[2 * j + 1] += (v[r][j] >> 8) & all;
+                f[2 * j] += v[r][j] & bef;
+                f[2 * j + 1] += (v[r][j] >> 8) & bef;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        part[sub][0][8 * c + j] = t[j];
+        part[sub][1][8 * c + j] = f[j];
+    }
+    __syncthreads();
+    // thread e: expert e is half (e >> 1) & 1 of dword 2 (e >> 2) + (e & 1)
+    const int d = 2 * (tid >> 2) + (tid & 1), sh = 8 * (tid & 2);
+    uint32_t ts = 0, fs = 0;
+#pragma unroll
+    for (int q = 0; q < kScSub; q++) {
+        ts += part[q][0][d];
+        fs += part[q][1][d];
+    }
+    tot = (int)((ts >> sh) & 0xffffu);
+    before = (int)((fs >> sh) & 0xffffu);
+}
+
 __global__ __launch_bounds__(256) void k_scatter(ScanArgs A) {
     __shared__ int tot[kMaxExperts], off[kMaxExperts + 1], ntile[kMaxExperts], toff[kMaxExperts + 1];
     __shared__ int boff[kMaxExperts];
+    __shared__ __align__(16) uint32_t part[kScSub][2][kMaxExperts / 2];
     const int tid = threadIdx.x, b = blockIdx.x;
     // this thread's first entry and shared-gate logit are loaded up front,
     // in flight with the totals and offsets
@@ -825,21 +885,20 @@ __global__ __launch_bounds__(256) void k_scatter(ScanArgs A) {
     const int ts = b * A.tpb + tid, ts1 = min(A.T, (b + 1) * A.tpb);
     float sga = 0.0f;
     if (A.shg && ts < ts1) sga = A.shg[(size_t)ts * A.ld_shg];
-    for (int e = tid; e < A.E; e += 256) {
-        if (A.inline_cols) {
-            const int32_t *cnt = A.blk_cnt + (size_t)e * A.nb;
-            int run = 0, mine = 0;
-            for (int bb = 0; bb < A.nb; bb++) {
-                if (bb == b) mine = run;
-                run += cnt[bb];
-            }
-            tot[e] = run;
-            boff[e] = mine;
-        } else {
-            tot[e] = A.tot[e];
-            boff[e] = A.blk_off[(size_t)e * A.nb + b];
-        }
-        ntile[e] = (tot[e] + A.tn - 1) / A.tn;
+    static_assert(kMaxExperts == 256, "one expert per thread");
+    int mine = 0, before = 0;
+    if (A.inline_cols) {
+        if (A.nb <= 2 * kScSub) scan_block_counts<2>(A.blk_cnt, A.nb, b, part, mine, before);
+        else if (A.nb <= 8 * kScSub) scan_block_counts<8>(A.blk_cnt, A.nb, b, part, mine, before);
+        else scan_block_counts<16>(A.blk_cnt, A.nb, b, part, mine, before);
+    } else if (tid < A.E) {
+        mine = A.tot[tid];
+        before = A.blk_off[(size_t)tid * A.nb + b];
+    }
+    if (tid < A.E) {
+        tot[tid] = mine;
+        boff[tid] = before;
+        ntile[tid] = (mine + A.tn - 1) / A.tn;
     }
     __syncthreads();
     if (tid < 64) wave_scan256(tot, A.E, off, &off[A.E]);
@@ -3116,7 +3175,8 @@ struct Scratch {
     size_t tile_cap;
     int32_t *topk_idx; float *topk_w; int32_t *rank;
     uint8_t *xq, *xs, *xs2;
-    int32_t *blk_cnt, *blk_off, *tot, *e_off, *perm, *pos, *row_tok;
+    uint8_t *blk_cnt;               // [routing blocks][kMaxExperts]
+    int32_t *blk_off, *tot, *e_off, *perm, *pos, *row_tok;
     float *row_w;
     int4 *tiles; int32_t *ntiles;
     uint8_t *hq, *hs, *hs2;
@@ -3209,7 +3269,7 @@ size_t carve_scratch(uint8_t *base, int max_T, int E, int D, int FF, int K, Scra
     const size_t o_idx = take(n * 4), o_w = take(n * 4), o_rank = take(n * 4);
     const size_t o_xq = take((size_t)max_T * D), o_xs = take((size_t)max_T * D / 32);
     const size_t o_xs2 = take((size_t)max_T * D / 32);
-    const size_t o_bc = take((size_t)c.nb_max * E * 4), o_bo = take((size_t)c.nb_max * E * 4);
+    const size_t o_bc = take((size_t)c.nb_max * kMaxExperts), o_bo = take((size_t)c.nb_max * E * 4);
     const size_t o_tot = take((size_t)E * 4);
     const size_t o_eo = take((size_t)(E + 1) * 4), o_perm = take(n * 4), o_pos = take(n * 4);
     const size_t o_rt = take(rows * 4), o_rw = take(rows * 4);
@@ -3226,7 +3286,7 @@ size_t carve_scratch(uint8_t *base, int max_T, int E, int D, int FF, int K, Scra
     c.topk_w = reinterpret_cast<float *>(b + o_w);
     c.rank = reinterpret_cast<int32_t *>(b + o_rank);
     c.xq = b + o_xq; c.xs = b + o_xs; c.xs2 = b + o_xs2;
-    c.blk_cnt = reinterpret_cast<int32_t *>(b + o_bc);
+    c.blk_cnt = b + o_bc;
     c.blk_off = reinterpret_cast<int32_t *>(b + o_bo);
     c.tot = reinterpret_cast<int32_t *>(b + o_tot);
     c.e_off = reinterpret_cast<int32_t *>(b + o_eo);

@@ -798,6 +798,31 @@ def test_router_logits_bf16_input_and_no_shared(dev):
     assert (np.abs(lg.cpu().numpy() - ref) / mag).max() <= 2e-6
 
 
+@pytest.mark.parametrize("T,E", [(257, 256), (513, 256), (1000, 5), (4112, 256), (8192, 256), (8193, 64), (8449, 256),
+                                 (12304, 9)])
+def test_scan_order(dev, T, E):
+    """The stable sorted order on both sides of the in-kernel scan's limit
+    (512 blocks of 16 tokens), at whole and ragged blocks and rounds of 256
+    blocks, with one expert that every token picks (counts of 16, the byte
+    sums' largest)."""
+    w = moe.MoEWeights.alloc(E, 2048, 512).fill_synthetic(3, -9, -5)
+    k = min(8, E)
+    layer = moe.MoELayer(T, n_expert=E, top_k=k)
+    layer.set_path(layer.PATH_SORTED)
+    g = torch.Generator(device=dev).manual_seed(T)
+    lg = torch.randn(T, E, device=dev, generator=g)
+    lg[:, E // 2] += 100.0
+    x = torch.randn(T, 2048, device=dev, generator=g)
+    layer.forward(w, x, lg)
+    torch.cuda.synchronize()
+    idx = layer.tap(moe.TAP_TOPK_IDX).flatten().long()
+    perm, pos, off = (layer.tap(t).long() for t in (moe.TAP_PERM, moe.TAP_POS, moe.TAP_EOFF))
+    assert torch.equal(perm, torch.sort(idx, stable=True).indices)
+    assert torch.equal(perm[pos], torch.arange(T * k, device=dev))
+    cnt = torch.bincount(idx, minlength=E)
+    assert cnt[E // 2] == T and torch.equal(off, torch.cat([cnt.new_zeros(1), cnt.cumsum(0)]))
+
+
 # every tile shape of the fp16 router at its edges: 257 rows (the last row
 # block takes a fifth tile) and row counts around a block, T at both sides of
 # each rule and with remainders
