@@ -2219,6 +2219,7 @@ struct SxArgs {
     int T, k, E;
     int discover;                          // 0: tiles from k_scatter
     int tn;                                // rows per discovered tile (<= kSkTok)
+    int sh8_first;                         // q8_0-split shared expert: first workgroup of its gate/up
 };
 
 __device__ __forceinline__ int sx_off(int r, int c) { return r * 2048 + ((c & ~15) | ((c ^ r) & 15)) * 16; }
@@ -2482,7 +2483,7 @@ __device__ __forceinline__ void skinny_expert(const GemmArgs &G, const GemmArgs 
 // Finds this workgroup's tile (expert e, sorted rows p0..p1) from the top-k
 // indices; false past the last tile.  ev / wv keep this thread's entries
 // for sx_gather.
-__device__ bool sx_find(const SxArgs &X, SxLds &L, int ti, int &e_out, int &p0_out, int &p1_out, int (&ev)[kSxEnt],
+__device__ __forceinline__ bool sx_find(const SxArgs &X, SxLds &L, int ti, int &e_out, int &p0_out, int &p1_out, int (&ev)[kSxEnt],
                         float (&wv)[kSxEnt]) {
     const int tid = threadIdx.x, wave = tid >> 6;
     const int n = X.T * X.k, E = X.E;
@@ -2531,7 +2532,7 @@ __device__ bool sx_find(const SxArgs &X, SxLds &L, int ti, int &e_out, int &p0_o
 // Fills L.tok / L.ws with the rows of the tile sx_find found and writes
 // their pos / perm.  It runs while the first weight step is in flight, so
 // its barriers wait on LDS only.
-__device__ void sx_gather(const SxArgs &X, SxLds &L, int e, int p0, int p1, const int (&ev)[kSxEnt],
+__device__ __forceinline__ void sx_gather(const SxArgs &X, SxLds &L, int e, int p0, int p1, const int (&ev)[kSxEnt],
                           const float (&wv)[kSxEnt]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = X.T * X.k;
@@ -2580,10 +2581,131 @@ __device__ void sx_gather(const SxArgs &X, SxLds &L, int e, int p0, int p1, cons
     lds_barrier();
 }
 
+// Gate/up, SwiGLU and int8 h of a q8_0-split shared expert for 32 tokens and
+// 32 rows of h, by a workgroup of the launch that streams the routed experts
+// (its down projection follows in k_combine_sh8): the work is too small for
+// launches of its own, and most of the routed tiles' run time leaves CUs idle
+// or waiting on memory.  8 waves split K (256 each); the wave's weights (4
+// row tiles x 4 K-pairs, codes and scales) are all in flight while the tile's
+// int8 x is staged in LDS.  Partial sums meet in LDS in wave order.
+// Layer, us at T = 17 / 40 / 128 / 256 / 512, Q8_0 shared and MXFP4 routed
+// experts: 115 / 136 / 166 / 177 / 122 with separate gate/up, shared gate/up
+// (61 us in 16 workgroups) and down kernels, or fat tiles from T = 257;
+// 50 / 58 / 83 / 87 / 109 this way.
+constexpr int kSh8Tok = 32;              // tokens per workgroup (two column tiles)
+constexpr int kSh8Sf = 66;               // floats per staged row of x scales
+static_assert(kSh8Tok == kSkTok && sizeof(float) * kSh8Tok * kSh8Sf <= sizeof(SxLds::h), "x and its scales fit L.x / L.h");
+static_assert(kSxW * 4 * (kSh8Tok / 16) * 64 * 16 <= sizeof(SxLds::x), "the partial sums fit L.x");
+__device__ __forceinline__ void sh8_gateup(const GemmArgs &A, SxLds &L, int tb, int rb) {
+    constexpr int KD = 2048, NKP = KD / 64, NKB = KD / 32, MF = 512, KPW = NKP / kSxW, NJ = kSh8Tok / 16;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = tb * kSh8Tok, mt0 = rb * 2, kp0 = wave * KPW;
+    u32x4 af[4][KPW], sf[4][KPW];        // gate mt0, mt0+1, up mt0, mt0+1
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        const uint8_t *W = a < 2 ? A.sa : A.sb;
+        const int mt = mt0 + (a & 1);
+#pragma unroll
+        for (int u = 0; u < KPW; u++) {
+            af[a][u] = *reinterpret_cast<const u32x4 *>(W + ((size_t)mt * NKP + kp0 + u) * 1024 + lane * 16);
+            sf[a][u] = *reinterpret_cast<const u32x4 *>(W + (size_t)MF * KD + (((size_t)mt * 4 + q) * NKB + 2 * (kp0 + u)) * 8);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {   // rows past the last token repeat it; never stored
+        const int r = tid >> 4, c = tid & 15;
+        const int t = min(t0 + r, A.T - 1);
+        u32x4 xv[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            xv[u] = *reinterpret_cast<const u32x4 *>(A.xq8 + (size_t)t * KD + (c + 16 * u) * 16);
+        const float4 sv = *reinterpret_cast<const float4 *>(A.xsf + (size_t)t * NKB + 4 * c);
+#pragma unroll
+        for (int u = 0; u < 8; u++) *reinterpret_cast<u32x4 *>(&L.x[sx_off(r, c + 16 * u)]) = xv[u];
+        float *d = reinterpret_cast<float *>(L.h) + r * kSh8Sf + 4 * c;
+        *reinterpret_cast<float2 *>(d) = make_float2(sv.x, sv.y);
+        *reinterpret_cast<float2 *>(d + 2) = make_float2(sv.z, sv.w);
+    }
+    lds_barrier();
+    v4f acc[4][NJ];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[a][j] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < KPW; u++) {
+        float2 dh[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            dh[j] = *reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(L.h) + (16 * j + n) * kSh8Sf + 2 * (kp0 + u));
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int kb = 2 * (kp0 + u) + h;
+            long bv[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const uint2 v = *reinterpret_cast<const uint2 *>(&L.x[sx_off(16 * j + n, 2 * kb + (q >> 1)) + (q & 1) * 8]);
+                bv[j] = (long)(((uint64_t)v.y << 32) | v.x);
+            }
+            v4i ci[4][NJ];
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                const long av = (long)(((uint64_t)af[a][u][2 * h + 1] << 32) | af[a][u][2 * h]);
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+                    ci[a][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv[j], v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
+            }
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                const uint32_t s01 = sf[a][u][2 * h], s23 = sf[a][u][2 * h + 1];
+                const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[a][j][i] = fmaf(q8_scaled(ci[a][j][i], w[i], -kQ8BiasF * w[i]), h ? dh[j].y : dh[j].x, acc[a][j][i]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();                       // every wave has read its x
+    v4f *red = reinterpret_cast<v4f *>(L.x);   // [wave][col tile][row tile][lane]
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) red[((wave * NJ + j) * 4 + a) * 64 + lane] = acc[a][j];
+    lds_barrier();
+    if (wave >= NJ) return;              // wave j finishes column tile j
+    v4f sum[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        sum[a] = red[(wave * 4 + a) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < kSxW; w++) sum[a] += red[((w * NJ + wave) * 4 + a) * 64 + lane];
+    }
+    float h[2][4];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[r][i] = silu(sum[r][i]) * sum[2 + r][i];
+    const int t = t0 + 16 * wave + n;
+    store_h_block(A, true, A.nrouted + t, t < A.T, mt0 * 16, q, lane, h);
+}
+
+// SH8: with the extra workgroups of a q8_0-split shared expert (a template
+// parameter: their registers cost the other layers 0.3 us).
+template <bool SH8>
 __global__ __launch_bounds__(64 * kSxW) void k_skinny_expert(GemmArgs G, GemmArgs Dn, SxArgs X) {
     __shared__ SxLds L;
     const int ti = blockIdx.x;
     int e, p0, p1;
+    if constexpr (SH8) {
+        if (ti >= X.sh8_first) {
+            sh8_gateup(G, L, (ti - X.sh8_first) / kShRb, (ti - X.sh8_first) % kShRb);
+            return;
+        }
+    }
     if (X.discover) {
         int ev[kSxEnt];
         float wv[kSxEnt];
@@ -3064,6 +3186,93 @@ __global__ __launch_bounds__(256) void k_combine(const uint16_t *__restrict__ dn
     }
 }
 
+// Combine with a q8_0-split shared expert on the one-kernel skinny path: 16
+// tokens x 64 columns per workgroup.  Each wave runs one row tile of the
+// shared down on the tokens' int8 h rows (the 16 blocks of k_gemm_expert_i8,
+// q36_engine.cu:2526-2618) while the routed rows' loads are in flight; the
+// results meet the thread that owns (token, 4 columns) in LDS and are added
+// last, weighted, as k_combine adds the shared row.  The rows are also staged
+// for the DNW tap, as the separate down kernel stages them.
+__global__ __launch_bounds__(256) void k_combine_sh8(GemmArgs A, const float *__restrict__ shg, int ld_shg, int k,
+                                                     void *out, int out_fmt) {
+    constexpr int KD = 512, NKP = KD / 64, NKB = KD / 32, DO = 2048;
+    __shared__ __align__(16) uint8_t sh[16 * KD];
+    __shared__ __align__(16) float ssf[16][kDlSfStride];
+    __shared__ __align__(16) float res[16][68];
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = blockIdx.x * 16, mt = blockIdx.y * 4 + wave;
+    u32x4 ac[NKP], as[NKP];
+#pragma unroll
+    for (int kp = 0; kp < NKP; kp++) {
+        ac[kp] = *reinterpret_cast<const u32x4 *>(A.sa + ((size_t)mt * NKP + kp) * 1024 + lane * 16);
+        as[kp] = *reinterpret_cast<const u32x4 *>(A.sa + (size_t)DO * KD + (((size_t)mt * 4 + q) * NKB + 2 * kp) * 8);
+    }
+    // rows past the last token repeat it; never stored
+    const int tk = tid >> 4, c4 = (tid & 15) * 4, t = min(t0 + tk, A.T - 1), col = blockIdx.y * 64 + c4;
+    uint2 hv[kMaxTopK];
+    uint32_t ev[kMaxTopK];
+#pragma unroll
+    for (int s = 0; s < kMaxTopK; s++)
+        if (s < k) {
+            const size_t p = (size_t)t * k + s;
+            hv[s] = *reinterpret_cast<const uint2 *>(A.dnh + p * DO + col);
+            ev[s] = A.dne[p * (DO / 16) + (col >> 4)];
+        }
+    const size_t ph = (size_t)A.nrouted + t;
+    const int hc = (tid & 15) * 2;
+    const u32x4 h0 = *reinterpret_cast<const u32x4 *>(A.bq + ph * KD + hc * 16);
+    const u32x4 h1 = *reinterpret_cast<const u32x4 *>(A.bq + ph * KD + hc * 16 + 16);
+    *reinterpret_cast<u32x4 *>(&sh[dl_boff(tk, hc)]) = h0;
+    *reinterpret_cast<u32x4 *>(&sh[dl_boff(tk, hc + 1)]) = h1;
+    ssf[tk][tid & 15] = A.bsf[ph * NKB + (tid & 15)];
+    const float wsh = 1.0f / (1.0f + expf(-shg[(size_t)t * ld_shg]));
+    lds_barrier();
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < NKB; kb++) {
+        const uint2 bv = *reinterpret_cast<const uint2 *>(&sh[dl_boff(n, 2 * kb + (q >> 1)) + (q & 1) * 8]);
+        const long b = (long)(((uint64_t)bv.y << 32) | bv.x);
+        const u32x4 f = ac[kb >> 1];
+        const long a = (kb & 1) ? (long)(((uint64_t)f[3] << 32) | f[2]) : (long)(((uint64_t)f[1] << 32) | f[0]);
+        const v4i ci = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
+        const float dh = ssf[n][kb];
+        const uint32_t s01 = as[kb >> 1][2 * (kb & 1)], s23 = as[kb >> 1][2 * (kb & 1) + 1];
+        const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] = fmaf(q8_scaled(ci[i], w[i], -kQ8BiasF * w[i]), dh, acc[i]);
+    }
+    *reinterpret_cast<v4f *>(&res[n][wave * 16 + 4 * q]) = acc;   // column n = token, rows 4q.. = columns
+    lds_barrier();
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kMaxTopK; s++)
+        if (s < k) {
+            const float sc = __uint_as_float((ev[s] - 14u) << 23);
+            a[0] += f16lo(hv[s].x) * sc;
+            a[1] += f16hi(hv[s].x) * sc;
+            a[2] += f16lo(hv[s].y) * sc;
+            a[3] += f16hi(hv[s].y) * sc;
+        }
+    const v4f r = *reinterpret_cast<const v4f *>(&res[tk][c4]);
+    const float v[4] = {r[0] * wsh, r[1] * wsh, r[2] * wsh, r[3] * wsh};
+    // the tap's staged row: one exponent per 16 columns (four lanes)
+    float m = max_quad(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    uint32_t eb = (__float_as_uint(m) >> 23) & 0xffu;
+    eb = eb == 255u ? 255u : eb < 15u ? 15u : eb > 254u ? 254u : eb;
+    const float mul = __uint_as_float((268u - eb) << 23);
+    if (t0 + tk >= A.T) return;
+    *reinterpret_cast<uint2 *>(A.dnh + ph * DO + col) = make_uint2(f16x2(v[0] * mul, v[1] * mul), f16x2(v[2] * mul, v[3] * mul));
+    if ((tid & 3) == 0) A.dne[ph * (DO / 16) + (col >> 4)] = (uint8_t)eb;
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[i] += v[i];
+    if (out_fmt == Q36MOE_FMT_F32)
+        *reinterpret_cast<float4 *>(static_cast<float *>(out) + (size_t)t * DO + col) = make_float4(a[0], a[1], a[2], a[3]);
+    else
+        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(out) + (size_t)t * DO + col) =
+            make_uint2(f32_to_bf16(a[0]) | (f32_to_bf16(a[1]) << 16), f32_to_bf16(a[2]) | (f32_to_bf16(a[3]) << 16));
+}
+
 // The staged down rows widened to f32 (the DNW debug tap).
 __global__ __launch_bounds__(256) void k_dn16_expand(const uint16_t *__restrict__ dnh, const uint8_t *__restrict__ dne,
                                                     int D, float *__restrict__ dst) {
@@ -3163,6 +3372,7 @@ struct Plan {
     GemmArgs ga, da;
     SxArgs sx;
     DirectArgs di;
+    const float *shg; int ld_shg;
     const void *out; int out_fmt;
 };
 
@@ -3601,7 +3811,11 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             break;
         case ST_GATEUP:
             if (P.fused) {
-                hipLaunchKernelGGL(k_skinny_expert, dim3(P.tiles), dim3(64 * kSxW), 0, s, P.ga, P.da, P.sx);
+                if (P.ga.shq8)
+                    hipLaunchKernelGGL(k_skinny_expert<true>, dim3(P.tiles + (T + kSh8Tok - 1) / kSh8Tok * kShRb),
+                                       dim3(64 * kSxW), 0, s, P.ga, P.da, P.sx);
+                else
+                    hipLaunchKernelGGL(k_skinny_expert<false>, dim3(P.tiles), dim3(64 * kSxW), 0, s, P.ga, P.da, P.sx);
             } else if (P.skinny) {
                 hipLaunchKernelGGL(k_skinny_gateup, dim3(P.tiles * 16), dim3(64 * kSkW), 0, s, P.ga);
                 if (P.ga.shq8)
@@ -3621,6 +3835,11 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
                                    s, P.da);
             break;
         case ST_COMBINE:
+            if (P.fused && P.da.shq8) {
+                hipLaunchKernelGGL(k_combine_sh8, dim3((T + 15) / 16, D / 64), dim3(256), 0, s, P.da, P.shg, P.ld_shg, K,
+                                   const_cast<void *>(P.out), P.out_fmt);
+                break;
+            }
             // small batches: 64-thread blocks, so the work spreads over more CUs
             hipLaunchKernelGGL(k_combine, dim3(T, T < 256 ? D / 512 : D / 2048), dim3(T < 256 ? 64 : 256), 0, s, c.dnh,
                                c.dne, P.fused && P.sx.discover ? nullptr : c.pos, T, K, D, P.has_sh,
@@ -3680,7 +3899,10 @@ static int launch_forward(const Scratch &c, Plan &P, int pm, const q36moe_weight
     // most kSkinnyRows rows, else fat tiles of up to kGdTok rows
     // the one-kernel skinny path (every matrix MXFP4) serves twice the rows
     // per expert: it beat fat tiles up to 512 tokens (T=384: 96 vs 103 us)
-    const bool fusable = !w->dn_q8 && !shq8;
+    // a q8_0-split shared expert rides along (its gate/up in extra workgroups
+    // of that launch, its down in the combine) where the tiles are found
+    // in-kernel; a forced path keeps the two kernels
+    const bool fusable = !w->dn_q8 && (!shq8 || (pm == 0 && n <= kSxDiscoverMax));
     const size_t skinny_rows = (size_t)(fusable ? kSxFusedRows : kSkinnyRows) * E;
     const bool skinny = pm == 4 || pm == 5 || (pm == 0 && (size_t)n <= skinny_rows);
     // skinny tiles in one kernel per tile (k_skinny_expert) when every
@@ -3696,6 +3918,7 @@ static int launch_forward(const Scratch &c, Plan &P, int pm, const q36moe_weight
     P = Plan{};
     P.T = T; P.has_sh = has_sh; P.direct = direct; P.skinny = skinny; P.fused = fused;
     P.tiles = tiles; P.nb = nb; P.out = out; P.out_fmt = out_fmt;
+    P.shg = shg; P.ld_shg = ld_shg;
     if (direct) {
         P.di = DirectArgs{logits, ld_logits, T, E, K, scale, x, x_fmt, shg, ld_shg,
                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
@@ -3727,12 +3950,13 @@ static int launch_forward(const Scratch &c, Plan &P, int pm, const q36moe_weight
         // rather than a second stream of the same weights, and no more tiles
         // than CUs (T=256: 100.5 -> 85.5 us)
         const int stn = (size_t)n <= (size_t)4 * E ? kSxTok : kSkTok;
-        P.sx = SxArgs{c.topk_idx, c.topk_w, shg, ld_shg, c.perm, c.pos, c.e_off, T, K, E,
-                      fused && n <= kSxDiscoverMax ? 1 : 0, stn};
+        P.sx = SxArgs{c.topk_idx, c.topk_w, shq8 ? nullptr : shg, ld_shg, c.perm, c.pos, c.e_off, T, K, E,
+                      fused && n <= kSxDiscoverMax ? 1 : 0, stn, 0};
         if (P.sx.discover) {   // grid for tiles of stn rows; no counts for a scatter
             P.ra.counts = 0;
-            int t = n / stn + (n < E ? n : E) + (has_sh ? (T + stn - 1) / stn : 0);
+            int t = n / stn + (n < E ? n : E) + (has_sh && !shq8 ? (T + stn - 1) / stn : 0);
             P.tiles = (t + 7) & ~7;
+            if (shq8) P.sx.sh8_first = P.tiles;
         }
     }
     bind_weights(P, w);

@@ -646,6 +646,42 @@ def test_forward_q8_shared(oracle, q8_shared_layer, which, T, path):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["mx", "both"])
+@pytest.mark.parametrize("T", [17, 31, 33, 48, 130, 257, 512, 513])
+def test_forward_q8_shared_small_batches(oracle, q8_shared_layer, which, T):
+    """The automatic path of small batches: the shared expert beside the
+    routed tiles, at whole and partial tiles of 16 and 32 tokens, both row
+    counts of the routed tiles and the path's limit (512 tokens)."""
+    _check_shared_q8(oracle, q8_shared_layer, which, T, 0, 1500 + T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [23, 200])
+def test_q8_shared_taps_and_replays(q8_shared_layer, T):
+    """The staged shared rows (DNW tap) are the shared term of the output,
+    bf16 output is the rounded f32 one, a strided shared gate gives the same
+    bits, and so does a second forward."""
+    import torch
+    from q36_amd import moe
+    dw = q8_shared_layer["mx"]
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, 2048, device="cuda", generator=g)
+    lg = torch.randn(T, 257, device="cuda", generator=g)
+    layer = moe.MoELayer(T)
+    y = layer.forward(dw, x, lg, lg[:, 256], out_dtype=torch.float32)
+    dn = layer.tap(moe.TAP_DNW)
+    yb = layer.forward(dw, x, lg, lg[:, 256].contiguous())
+    torch.cuda.synchronize()
+    assert torch.equal(yb, y.to(torch.bfloat16))
+    routed = layer.forward(dw, x, lg, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    sh = dn[T * 8:]
+    # the tap rounds to 11 bits below each 16-column maximum
+    bar = sh.view(T, -1, 16).abs().amax(2, keepdim=True).expand(-1, -1, 16).reshape(T, -1) * 2.0 ** -10
+    assert ((y - routed - sh).abs() <= bar + 1e-6 * y.abs().max()).all()
+
+
+@pytest.mark.gpu
 def test_q8_shared_refusals(q8_shared_layer):
     import torch
     from q36_amd import moe
