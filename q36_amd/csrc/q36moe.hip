@@ -515,6 +515,9 @@ __device__ __forceinline__ float f16hi(uint32_t d) { return (float)__builtin_bit
 constexpr int kQ8Bias = 0x4B400000;
 constexpr float kQ8BiasF = 12582912.0f;
 __device__ __forceinline__ float q8_scaled(int r, float w, float nwb) { return fmaf(__int_as_float(r), w, nwb); }
+// -12582912 * w; as an fma the f16 operand needs no conversion of its own
+// (v_fma_mix_f32), which a multiply would
+__device__ __forceinline__ float q8_nwb(float w) { return fmaf(-kQ8BiasF, w, 0.0f); }
 
 struct RouteArgs {
     const float *logits; int ld; int T; int E; int k; float scale;
@@ -1307,50 +1310,59 @@ __device__ __forceinline__ void body(const GemmArgs &A, Lds &L, const uint8_t *W
 // takes tokens 64w..64w+63 (4 column tiles) against the 4 row tiles over all
 // of K = 2048, so each weight fragment loaded feeds 4 MFMAs (the weights,
 // 2 MiB for gate + up, stay in L2).  Each block's integer result is scaled
-// and added in fp32.  The epilogue is the routed kernels': SwiGLU and the
-// int8 quantisation of h into the token's shared row.
+// and added in fp32: two fmas per output and 32-block, which bound the body
+// (with the f16 scales' bias products shared by 4 column tiles, 9 VALU
+// instructions per MFMA).  The wave's x, 128 bytes of each of its rows (two
+// K-pairs) per stage, goes to its own LDS by direct-to-LDS loads, two stages,
+// no barrier; loaded in operand order, whose neighbouring lanes lie in
+// different rows, x kept the address unit busy for a lane a cycle (768 cycles
+// per K-pair and wave, against 1280 of scaling on each SIMD): layer of 4006
+// tokens 276 us, 258 this way.
+// The epilogue is the routed kernels': SwiGLU and the int8 quantisation of h
+// into the token's shared row.
 constexpr int kShCt = 4;                 // column tiles per wave
 constexpr int kShTok = 4 * 16 * kShCt;   // tokens per workgroup
 constexpr int kShRb = 512 / 32;          // 32-row blocks of d_ff
+constexpr int kShStage = 64 * 128 + 64 * 16;   // bytes per wave and stage: x rows, their scales
+constexpr int kShLds = 4 * 2 * kShStage;
 
 // Operands of one K-pair (two 32-blocks) of the shared gate/up body.
 struct ShKp {
     u32x4 af[4], sf[4];      // weight codes and f16 scales of the 4 row tiles
-    uint2 bx[kShCt][2];      // x codes of the column tiles, both blocks
-    float2 dh[kShCt];        // their fp32 scales
 };
 
 // Workgroup (token block tb, 32-row block rb) of the shared gate/up.
-__device__ __forceinline__ void shared_gateup_q8_body(const GemmArgs &A, int tb, int rb) {
-    constexpr int KD = 2048, NKP = KD / 64, NKB = KD / 32, MF = 512;
+__device__ __forceinline__ void shared_gateup_q8_body(const GemmArgs &A, int tb, int rb, uint8_t *lds) {
+    constexpr int KD = 2048, NKP = KD / 64, NKB = KD / 32, MF = 512, NST = NKP / 2;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = tb * kShTok + wave * 16 * kShCt;   // this wave's first token
     const int mt0 = rb * 2;                            // first row tile of the 32-row block
     if (t0 >= A.T) return;                             // wave-uniform; no barrier follows
-    const int8_t *xr[kShCt];
-    const float *xs[kShCt];
+    uint8_t *st = lds + wave * 2 * kShStage;
+    const int nt = A.T - t0;                           // rows past the end repeat the last token; never stored
+    const __amdgpu_buffer_rsrc_t rx = dma_src(A.xq8 + (size_t)t0 * KD), rs = dma_src(A.xsf + (size_t)t0 * NKB);
+    const __amdgpu_buffer_rsrc_t rg = dma_src(A.sa), ru = dma_src(A.sb);
+    uint32_t xo[8];
 #pragma unroll
-    for (int j = 0; j < kShCt; j++) {
-        // padding columns repeat the last token; never stored
-        const int t = min(t0 + 16 * j + n, A.T - 1);
-        xr[j] = A.xq8 + (size_t)t * KD;
-        xs[j] = A.xsf + (size_t)t * NKB;
+    for (int i = 0; i < 8; i++) {
+        const int m = 4 * i + (lane >> 4), sl = (lane & 15) ^ (m & 7);
+        xo[i] = (uint32_t)min(2 * m + (sl >> 3), nt - 1) * KD + (sl & 7) * 16;
     }
+    const uint32_t so = (uint32_t)min(lane, nt - 1) * (NKB * 4);
+    auto stage = [&](int s) {
+        uint8_t *d = st + (s & 1) * kShStage;
+#pragma unroll
+        for (int i = 0; i < 8; i++) dma16(rx, xo[i] + s * 128, d + i * 1024);
+        dma16(rs, so + s * 16, d + 64 * 128);
+    };
     auto load = [&](int kp, ShKp &o) {
 #pragma unroll
         for (int a = 0; a < 4; a++) {
-            const uint8_t *W = a < 2 ? A.sa : A.sb;
             const int mt = mt0 + (a & 1);
-            o.af[a] = *reinterpret_cast<const u32x4 *>(W + ((size_t)mt * NKP + kp) * 1024 + lane * 16);
-            o.sf[a] = *reinterpret_cast<const u32x4 *>(W + (size_t)MF * KD + (((size_t)mt * 4 + q) * NKB + 2 * kp) * 8);
-        }
-        // x K 64kp + 8q..+7 (block 2kp) and 64kp + 32 + 8q..+7 (block 2kp+1)
-#pragma unroll
-        for (int j = 0; j < kShCt; j++) {
-            o.bx[j][0] = *reinterpret_cast<const uint2 *>(xr[j] + 64 * kp + 8 * q);
-            o.bx[j][1] = *reinterpret_cast<const uint2 *>(xr[j] + 64 * kp + 32 + 8 * q);
-            o.dh[j] = *reinterpret_cast<const float2 *>(xs[j] + 2 * kp);
+            o.af[a] = __builtin_amdgcn_raw_buffer_load_b128(a < 2 ? rg : ru, (uint32_t)lane * 16, (mt * NKP + kp) * 1024, 0);
+            o.sf[a] = __builtin_amdgcn_raw_buffer_load_b128(a < 2 ? rg : ru, (uint32_t)q * (NKB * 8),
+                                                            MF * KD + mt * (4 * NKB * 8) + kp * 16, 0);
         }
     };
     v4f acc[4][kShCt];   // gate mt0, mt0+1, up mt0, mt0+1 x column tiles
@@ -1358,31 +1370,74 @@ __device__ __forceinline__ void shared_gateup_q8_body(const GemmArgs &A, int tb,
     for (int a = 0; a < 4; a++)
 #pragma unroll
         for (int j = 0; j < kShCt; j++) acc[a][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    ShKp cur, nxt;
-    load(0, cur);
-#pragma unroll 1
-    for (int kp = 0; kp < NKP; kp++) {
-        if (kp + 1 < NKP) load(kp + 1, nxt);   // in flight while this pair computes
+    struct Frag {        // the column tiles' x of a K-pair: codes of both blocks, scales
+        long b[2][kShCt];
+        float2 d[kShCt];
+    };
+    auto read = [&](const uint8_t *d, int u, Frag &f) {   // K-pair u of the stage in slot d
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+        for (int j = 0; j < kShCt; j++) {
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const long av = (long)(((uint64_t)cur.af[a][2 * h + 1] << 32) | cur.af[a][2 * h]);
-                const uint32_t s01 = cur.sf[a][2 * h], s23 = cur.sf[a][2 * h + 1];
-                const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
-                float nw[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) nw[i] = -kQ8BiasF * w[i];
-#pragma unroll
-                for (int j = 0; j < kShCt; j++) {
-                    const long b = (long)(((uint64_t)cur.bx[j][h].y << 32) | cur.bx[j][h].x);
-                    const v4i ci = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, b, v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
-                    const float dhh = h ? cur.dh[j].y : cur.dh[j].x;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[a][j][i] = fmaf(q8_scaled(ci[i], w[i], nw[i]), dhh, acc[a][j][i]);
-                }
+            for (int h = 0; h < 2; h++) {
+                const uint2 v = *reinterpret_cast<const uint2 *>(d + gd_boff(16 * j + n, 4 * u + 2 * h + (q >> 1)) + (q & 1) * 8);
+                f.b[h][j] = (long)(((uint64_t)v.y << 32) | v.x);
             }
-        cur = nxt;
+            f.d[j] = *reinterpret_cast<const float2 *>(d + 64 * 128 + (16 * j + n) * 16 + u * 8);
+        }
+    };
+    auto compute = [&](const Frag &f, const ShKp &o) {
+        v4i ci[2][kShCt];
+        // block (h, row tile a) = group g: its MFMAs run while group g-1 is scaled
+        static_for<0, 9>([&](auto G) {
+            constexpr int g = decltype(G)::value;
+            if constexpr (g < 8) {
+                constexpr int h = g >> 2, a = g & 3;
+                const long av = (long)(((uint64_t)o.af[a][2 * h + 1] << 32) | o.af[a][2 * h]);
+#pragma unroll
+                for (int j = 0; j < kShCt; j++)
+                    ci[g & 1][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, f.b[h][j], v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
+            }
+            if constexpr (g > 0) {
+                constexpr int h = (g - 1) >> 2, a = (g - 1) & 3;
+                const uint32_t s01 = o.sf[a][2 * h], s23 = o.sf[a][2 * h + 1];
+                const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float nw = q8_nwb(w[i]);
+#pragma unroll
+                    for (int j = 0; j < kShCt; j++)
+                        acc[a][j][i] = fmaf(q8_scaled(ci[(g - 1) & 1][j][i], w[i], nw), h ? f.d[j].y : f.d[j].x, acc[a][j][i]);
+                }
+                auto &ac = acc;
+#pragma unroll
+                for (int j = 0; j < kShCt; j++) asm volatile("" : "+v"(ac[a][j]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    ShKp w0, w1;
+    Frag f;
+    stage(0);
+    load(0, w0);
+#pragma unroll 1
+    for (int s = 0; s < NST; s++) {
+        const uint8_t *d = st + (s & 1) * kShStage;
+        // everything issued so far: this stage's x (a stage ago) and its first
+        // K-pair's weights (a K-pair ago)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        // x is read before the next stage's loads go out: the compiler waits
+        // for every direct-to-LDS load issued before an LDS read
+        read(d, 0, f);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 1 < NST) stage(s + 1);   // its slot was last read in stage s - 1
+        load(2 * s + 1, w1);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(f, w0);
+        load(s + 1 < NST ? 2 * s + 2 : 0, w0);   // past the end: not used
+        __builtin_amdgcn_sched_barrier(0);
+        read(d, 1, f);
+        compute(f, w1);
     }
 #pragma unroll
     for (int j = 0; j < kShCt; j++) {
@@ -1398,8 +1453,9 @@ __device__ __forceinline__ void shared_gateup_q8_body(const GemmArgs &A, int tb,
 
 // Stand-alone launch (skinny-tile layers); fat-tile layers run the same
 // body in k_gateup_dma's first workgroups, beside the routed tiles.
-__global__ __launch_bounds__(256) void k_shared_gateup_q8(GemmArgs A) {
-    shared_gateup_q8_body(A, blockIdx.x, blockIdx.y);
+__global__ __launch_bounds__(256, 2) void k_shared_gateup_q8(GemmArgs A) {
+    __shared__ __align__(16) uint8_t lds[kShLds];
+    shared_gateup_q8_body(A, blockIdx.x, blockIdx.y, lds);
 }
 
 __global__ __launch_bounds__(256, 2) void k_gateup_dma(GemmArgs A) {
@@ -1410,7 +1466,8 @@ __global__ __launch_bounds__(256, 2) void k_gateup_dma(GemmArgs A) {
     // routed tiles
     const int bid = (int)blockIdx.x - A.sh_wgs;
     if (bid < 0) {
-        shared_gateup_q8_body(A, (int)blockIdx.x / kShRb, (int)blockIdx.x % kShRb);
+        static_assert(kShLds <= sizeof(gdma::Lds), "the shared body stages in the routed one's LDS");
+        shared_gateup_q8_body(A, (int)blockIdx.x / kShRb, (int)blockIdx.x % kShRb, reinterpret_cast<uint8_t *>(&L));
         return;
     }
     // tiles in reverse list order: k_scatter lists the routed tiles in
