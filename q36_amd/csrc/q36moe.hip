@@ -23,7 +23,7 @@
 //              token order (q36_engine.cu:3393-3401).
 // q8_0-split matrices (the reference's requantised k-quant experts and its
 // Q8_0 shared expert) run on int8 MFMA with per-32 scales: down_q8_tile in
-// k_down_lds<true>, the Q8 branches of k_direct_down<true> and
+// k_down_lds<1> and <2>, the Q8 branches of k_direct_down<true> and
 // k_direct_gateup<true, *>, and the shared gate/up body (k_shared_gateup_q8,
 // or the leading workgroups of k_gateup_dma).  In front of the boundary:
 // k_router_f32 / k_router_f16 (router logits) and k_add_rmsnorm_quant (the
@@ -1966,50 +1966,53 @@ constexpr int kDlRows = 128;             // B rows staged per chunk
 // dne; the combine multiplies back by 2^(eb - 141).  Half the bytes of an
 // f32 staging (which the reference uses, q36_engine.cu:3451-3463) for a
 // rounding of 2^-11 of each staged value.
-__device__ __forceinline__ void store_dn16(const GemmArgs &A, int p, int g, int q, bool valid, float v0, float v1,
-                                           float v2, float v3) {
-    float a = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
-    a = max_rows4(a);
-    uint32_t eb = (__float_as_uint(a) >> 23) & 0xffu;
-    eb = eb == 255u ? 255u : eb < 15u ? 15u : eb > 254u ? 254u : eb;
-    const float mul = __uint_as_float((268u - eb) << 23);
-    if (valid) {
-        const uint32_t lo = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v0 * mul)) |
-                            ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v1 * mul)) << 16);
-        const uint32_t hi = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v2 * mul)) |
-                            ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v3 * mul)) << 16);
-        *reinterpret_cast<uint2 *>(A.dnh + (size_t)p * A.ldo + g * 16 + 4 * q) = make_uint2(lo, hi);
-        if (q == 0) A.dne[(size_t)p * (A.ldo / 16) + g] = (uint8_t)eb;
-    }
+__device__ __forceinline__ uint2 dn16_pack(float v0, float v1, float v2, float v3) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
+    const f16x2v lo = __builtin_convertvector((f32x2){v0, v1}, f16x2v), hi = __builtin_convertvector((f32x2){v2, v3}, f16x2v);
+    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+}
+// v * 2^(141 - eb) times the routing weight w for a group whose maximum |v| * |w|
+// is a: the multiplier (w folded into the power of two, exact) and eb.
+__device__ __forceinline__ float dn16_scale(float a, float w, uint32_t &eb) {
+    eb = max((__float_as_uint(a) >> 23) & 0xffu, 15u);
+    return w * __uint_as_float((268u - eb) << 23);
 }
 
-// store_dn16 for the 4 row tiles mt0 .. mt0+3 (64 columns) of one MFMA
-// column tile at once: one maximum and one exponent for all 64 (written to
-// each of the 4 groups' exponent bytes), and the routing weight w folded into
-// the scale multiply.  f16 holds every value within 2^-29 of the group
-// maximum at full relative precision, so the wider group rounds the same.
-__device__ __forceinline__ void store_dn16x4(const GemmArgs &A, int p, int mt0, int q, bool valid, const v4f (&c)[4],
-                                             float w) {
+// The 4 row tiles mt0 .. mt0+3 (64 columns) of one MFMA column tile at once
+// (column n = row row(n), n < nr valid): one maximum and one exponent for all
+// 64 (written to each of the 4 groups' exponent bytes), and the routing weight
+// w folded into the scale multiply.  f16 holds every value within 2^-29 of the
+// group maximum at full relative precision, so the wider group rounds the
+// same.  The 16 rows are gathered in the wave's own 16 x 144 bytes of LDS and
+// leave as 16-byte stores whose 8 neighbouring lanes cover a row's 128 bytes:
+// in MFMA result order neighbouring lanes lie in different rows, and the
+// address unit takes such a store lane by lane (8 bytes a lane: down kernel of
+// 4096 tokens 86 us, 74 this way; layer 215.6 -> 202.4 us at 4000 tokens).
+constexpr int kDnT = 144;      // bytes per gathered row (128 and a pad against bank conflicts)
+template <class Row>
+__device__ __forceinline__ void store_dn16x4(const GemmArgs &A, int nr, int mt0, int q, int n, const v4f (&c)[4], float w,
+                                             uint8_t *ts, Row &&row) {
     float a = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; i++)
         a = fmaxf(a, fmaxf(fmaxf(fabsf(c[i][0]), fabsf(c[i][1])), fmaxf(fabsf(c[i][2]), fabsf(c[i][3]))));
-    a = max_rows4(a);
-    a *= fabsf(w);
-    uint32_t eb = (__float_as_uint(a) >> 23) & 0xffu;
-    eb = eb == 255u ? 255u : eb < 15u ? 15u : eb > 254u ? 254u : eb;
-    const float wm = w * __uint_as_float((268u - eb) << 23);
-    if (valid) {
+    uint32_t eb;
+    const float wm = dn16_scale(max_rows4(a) * fabsf(w), w, eb);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t lo = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(c[i][0] * wm)) |
-                                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(c[i][1] * wm)) << 16);
-            const uint32_t hi = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(c[i][2] * wm)) |
-                                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(c[i][3] * wm)) << 16);
-            *reinterpret_cast<uint2 *>(A.dnh + (size_t)p * A.ldo + (mt0 + i) * 16 + 4 * q) = make_uint2(lo, hi);
-        }
-        if (q == 0) *reinterpret_cast<uint32_t *>(A.dne + (size_t)p * (A.ldo / 16) + mt0) = eb * 0x01010101u;
+    for (int i = 0; i < 4; i++)
+        *reinterpret_cast<uint2 *>(ts + n * kDnT + i * 32 + q * 8) =
+            dn16_pack(c[i][0] * wm, c[i][1] * wm, c[i][2] * wm, c[i][3] * wm);
+    if (q == 0 && n < nr) *reinterpret_cast<uint32_t *>(A.dne + (size_t)row(n) * (A.ldo / 16) + mt0) = eb * 0x01010101u;
+    route_sync();
+    const int lane = 16 * q + n;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int r = 8 * u + (lane >> 3), ch = lane & 7;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(ts + r * kDnT + ch * 16);
+        if (r < nr) *reinterpret_cast<u32x4 *>(A.dnh + (size_t)row(r) * A.ldo + mt0 * 16 + ch * 8) = v;
     }
+    route_sync();
 }
 
 // byte offset of (row r, 16-byte chunk c) of a staged h row: rows of 512 B,
@@ -2041,113 +2044,180 @@ __device__ __forceinline__ void stage_h_rows(const uint8_t *bq, int c0, int nr, 
 // fragment read (16 B each) start in 16 distinct bank groups.
 constexpr int kDlSfStride = 20;
 
-// Down projection of one routed tile whose expert is in the q8_0-split
-// layout (k_gemm_expert_i8, q36_engine.cu:2526-2618): int8 h rows with fp32
-// scales against int8 weights with f16 scales.  Each 32-block is one
-// v_mfma_i32_16x16x32_i8 whose exact integer result is scaled by the
-// weight row's f16 scale times the h row's fp32 scale and accumulated in
-// fp32 (two fmas per output and block, q8_scaled).  The wave's 4 row tiles
-// run as 4 passes over the staged B (codes and fp32 scales of one row tile
-// are 160 VGPRs); B is staged once per chunk, as in the MXFP4 body.  Each
-// pass is software-pipelined by one block: a block's scaling overlaps the
-// next block's MFMA.
-__device__ __forceinline__ void down_q8_tile(const GemmArgs &A, const uint8_t *W, int p0, int p1, int rb, uint8_t *sb,
-                                             float (*ssf)[kDlSfStride], float *ws) {
-    constexpr int KD = 512, NKP = KD / 64, NKB = KD / 32;
+// Down projection of up to 64 rows of one tile whose expert is in the
+// q8_0-split layout (k_gemm_expert_i8, q36_engine.cu:2526-2618): int8 h rows
+// with fp32 scales against int8 weights with f16 scales.  Each 32-block is
+// one v_mfma_i32_16x16x32_i8 whose exact integer result is scaled by the
+// weight row's f16 scale times the h row's fp32 scale and accumulated in fp32
+// (two fmas per output and block, q8_scaled): VALU issue bounds the kernel on
+// large tiles, the weight stream on small ones.  The wave's 4 row tiles run as
+// 4 passes, each against all NJ column tiles of the chunk: the f16 scale's
+// bias product is shared by NJ MFMAs, and the weights are used up K-pair by
+// K-pair, so they stream through a ring of RD K-pairs that runs across the
+// passes and whose first loads go out before h is staged.  h fragments are
+// read from LDS FD - 1 blocks ahead; a block's scaling overlaps the next
+// block's MFMAs.  Results are gathered in LDS over the passes and leave as
+// whole 128-byte row pieces.  Layer with int8 routed and shared downs, us at
+// 513 / 1531 / 4000 tokens: 161 / 204 / 388 with one row tile's weights and
+// widened scales held in registers against one column tile at a time, each
+// row tile stored as it was done; 145 / 183 / 356 this way.
+constexpr int kDq8Rows = 64;
+constexpr int kDq8Gt = kDq8Rows * (128 + 4);   // bytes of a wave's gathered results
+template <int NJ>
+__device__ __forceinline__ void down_q8_chunk(const GemmArgs &A, const uint8_t *W, int mt0, int c0, int nr, uint8_t *sb,
+                                              float (*ssf)[kDlSfStride], float *ws, uint8_t *gt) {
+    constexpr int KD = 512, NKP = KD / 64, NKB = KD / 32, RD = 4, FD = 4;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint8_t *Wsc = W + (size_t)2048 * KD;   // f16 scales after the codes
-    const int mt0 = (rb * kDlW + wave) * kDlRT;
-    for (int c0 = p0; c0 < p1; c0 += kDlRows) {
-        const int nr = min(kDlRows, p1 - c0);
-        if (c0 != p0) __syncthreads();   // previous chunk fully read
-        stage_h_rows(A.bq, c0, nr, sb);
-        for (int c = tid; c < nr; c += 64 * kDlW) {
-            const float4 *src = reinterpret_cast<const float4 *>(A.bsf + (size_t)(c0 + c) * NKB);
+    const __amdgpu_buffer_rsrc_t rw = dma_src(W);
+    struct Kp { u32x4 c, s; } ring[RD];       // codes; f16 scales of rows 4q..4q+3, both blocks
+    auto load = [&](int u, Kp &o) {           // K-pair u & 7 of row tile mt0 + u / 8
+        const int mt = mt0 + u / NKP, kp = u % NKP;
+        o.c = __builtin_amdgcn_raw_buffer_load_b128(rw, (uint32_t)lane * 16, (mt * NKP + kp) * 1024, 0);
+        o.s = __builtin_amdgcn_raw_buffer_load_b128(rw, (uint32_t)q * (NKB * 8), 2048 * KD + mt * (4 * NKB * 8) + kp * 16, 0);
+    };
 #pragma unroll
-            for (int u = 0; u < 4; u++) *reinterpret_cast<float4 *>(&ssf[c][4 * u]) = src[u];
-            ws[c] = A.row_w[c0 + c];
+    for (int r = 0; r < RD; r++) load(r, ring[r]);
+    __builtin_amdgcn_sched_barrier(0);
+    stage_h_rows(A.bq, c0, nr, sb);
+    if (tid < 4 * nr)
+        *reinterpret_cast<float4 *>(&ssf[tid >> 2][4 * (tid & 3)]) =
+            *reinterpret_cast<const float4 *>(A.bsf + (size_t)(c0 + (tid >> 2)) * NKB + 4 * (tid & 3));
+    if (tid < nr) ws[tid] = A.row_w[c0 + tid];
+    __syncthreads();
+    // h K 32kb + 8q..+7 of row n = half q & 1 of chunk 2kb + q / 2 (dl_boff);
+    // column tile j and K half add constants.  Rows past nr hold whatever was
+    // staged there before; they are never stored.
+    const uint8_t *hb[4][2];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) hb[k][h] = sb + dl_boff(n, 4 * k + 2 * h + (q >> 1)) + (q & 1) * 8;
+    const float *db = ssf[n];
+    struct Frag { uint2 b[NJ]; float d[NJ]; } fr[FD];
+    auto read = [&](int k4, int k, int h, Frag &f) {   // 32-block 2 * (4 k4 + k) + h
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            f.b[j] = *reinterpret_cast<const uint2 *>(hb[k][h] + j * 16 * 512 + k4 * 256);
+            f.d[j] = db[j * 16 * kDlSfStride + 8 * k4 + 2 * k + h];
         }
-        __syncthreads();
-        const int ntt = (nr + 15) >> 4;
+    };
+#pragma unroll
+    for (int b = 0; b < FD - 1; b++) read(0, b >> 1, b & 1, fr[b]);
 #pragma unroll 1
-        for (int ps = 0; ps < kDlRT; ps++) {
-            const int mt = mt0 + ps;
-            u32x4 ac[NKP];
-            float dw[NKB][4];   // f16 scales of rows 4q..4q+3, widened once per pass
-            float ndw[NKB][4];  // -12582912 * dw (exact)
+    for (int ps = 0; ps < kDlRT; ps++) {
+        v4f acc[NJ];
 #pragma unroll
-            for (int kp = 0; kp < NKP; kp++) {
-                ac[kp] = *reinterpret_cast<const u32x4 *>(W + ((size_t)mt * NKP + kp) * 1024 + lane * 16);
-                const u32x4 sv = *reinterpret_cast<const u32x4 *>(Wsc + (((size_t)mt * 4 + q) * NKB + 2 * kp) * 8);
+        for (int j = 0; j < NJ; j++) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k4 = 0; k4 < NKP / RD; k4++) {
+            v4i ci[2][NJ];
+            // step = 32-block kb of the half: its MFMAs, then the scaling of
+            // the block before
+            static_for<0, 2 * RD + 1>([&](auto S) {
+                constexpr int kb = decltype(S)::value;
+                auto &ac = acc;
+                if constexpr (kb < 2 * RD) {
+                    constexpr int r = kb >> 1, h = kb & 1;
+                    const long a = (long)(((uint64_t)ring[r].c[2 * h + 1] << 32) | ring[r].c[2 * h]);
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    dw[2 * kp + h][0] = f16lo(sv[2 * h]);
-                    dw[2 * kp + h][1] = f16hi(sv[2 * h]);
-                    dw[2 * kp + h][2] = f16lo(sv[2 * h + 1]);
-                    dw[2 * kp + h][3] = f16hi(sv[2 * h + 1]);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) ndw[2 * kp + h][i] = -kQ8BiasF * dw[2 * kp + h][i];
-                }
-            }
-            for (int j = 0; j < ntt; j++) {
-                // padding columns read row 0 of the chunk; never stored
-                const int r = j * 16 + n < nr ? j * 16 + n : 0;
-                float dh[NKB];
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const float4 v = *reinterpret_cast<const float4 *>(&ssf[r][4 * u]);
-                    dh[4 * u] = v.x; dh[4 * u + 1] = v.y; dh[4 * u + 2] = v.z; dh[4 * u + 3] = v.w;
-                }
-                // all 16 B fragments read up front (one LDS latency per column
-                // tile): lane (column n, group q) holds h K 32kb + 8q..+7 =
-                // half q&1 of chunk 2kb + q/2
-                uint2 bv[NKB];
-#pragma unroll
-                for (int kb = 0; kb < NKB; kb++)
-                    bv[kb] = *reinterpret_cast<const uint2 *>(&sb[dl_boff(r, 2 * kb + (q >> 1)) + (q & 1) * 8]);
-                v4f acc = {0.f, 0.f, 0.f, 0.f};
-                v4i prev;
-#pragma unroll
-                for (int kb = 0; kb < NKB; kb++) {
-                    const long b = (long)(((uint64_t)bv[kb].y << 32) | bv[kb].x);
-                    const u32x4 f = ac[kb >> 1];
-                    const long a = (kb & 1) ? (long)(((uint64_t)f[3] << 32) | f[2]) : (long)(((uint64_t)f[1] << 32) | f[0]);
-                    const v4i ci = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
-                    if (kb > 0) {   // the previous block, while this one's MFMA runs
-#pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            acc[i] = fmaf(q8_scaled(prev[i], dw[kb - 1][i], ndw[kb - 1][i]), dh[kb - 1], acc[i]);
+                    for (int j = 0; j < NJ; j++) {
+                        const uint2 bv = fr[kb % FD].b[j];
+                        const long b = (long)(((uint64_t)bv.y << 32) | bv.x);
+                        ci[kb & 1][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
                     }
-                    prev = ci;
-                    // one block per scheduling group: left alone, the compiler
-                    // issues every block's MFMA first and holds all the results
-                    asm volatile("" : "+v"(acc));
-                    __builtin_amdgcn_sched_barrier(0);
                 }
+                if constexpr (kb > 0) {
+                    constexpr int pb = kb - 1, r = pb >> 1, h = pb & 1;
+                    const uint32_t s01 = ring[r].s[2 * h], s23 = ring[r].s[2 * h + 1];
+                    const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    acc[i] = fmaf(q8_scaled(prev[i], dw[NKB - 1][i], ndw[NKB - 1][i]), dh[NKB - 1], acc[i]);
-                {
-                    const float w = ws[r];
-                    store_dn16(A, c0 + j * 16 + n, mt, q, j * 16 + n < nr, acc[0] * w, acc[1] * w, acc[2] * w,
-                               acc[3] * w);
+                    for (int i = 0; i < 4; i++) {
+                        const float nw = q8_nwb(w[i]);
+#pragma unroll
+                        for (int j = 0; j < NJ; j++)
+                            acc[j][i] = fmaf(q8_scaled(ci[pb & 1][j][i], w[i], nw), fr[pb % FD].d[j], acc[j][i]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) asm volatile("" : "+v"(ac[j]));
+                    // K-pair r is used up: its slot takes the one RD ahead
+                    if constexpr (h == 1) {
+                        const int u = ps * NKP + k4 * RD + r + RD;
+                        load(u < kDlRT * NKP ? u : 0, ring[r]);   // past the end: not used
+                    }
                 }
-            }
+                // and its fragments' place takes block kb + FD - 1 (of the
+                // next pass past the last)
+                if constexpr (kb < 2 * RD) {
+                    constexpr int nb = kb + FD - 1;
+                    read((k4 + (nb >> 3)) & 1, (nb >> 1) & 3, nb & 1, fr[nb % FD]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+        // 16 columns of the wave's 64: gathered in LDS (16-byte chunks XORed
+        // with the row) with the group's exponent byte behind the rows
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int r = j * 16 + n;
+            const float w = ws[r];
+            uint32_t eb;
+            const float wm = dn16_scale(max_rows4(fmaxf(fmaxf(fabsf(acc[j][0]), fabsf(acc[j][1])),
+                                                        fmaxf(fabsf(acc[j][2]), fabsf(acc[j][3])))) * fabsf(w), w, eb);
+            *reinterpret_cast<uint2 *>(gt + r * 128 + (((2 * ps + (q >> 1)) ^ (r & 7)) << 4) + (q & 1) * 8) =
+                dn16_pack(acc[j][0] * wm, acc[j][1] * wm, acc[j][2] * wm, acc[j][3] * wm);
+            if (q == 0) gt[kDq8Rows * 128 + r * 4 + ps] = (uint8_t)eb;
+        }
+    }
+    // stored as 16 bytes a lane, 8 neighbouring lanes to a row's 128 bytes, as
+    // in store_dn16x4
+    route_sync();
+    if (lane < nr)
+        *reinterpret_cast<uint32_t *>(A.dne + (size_t)(c0 + lane) * (A.ldo / 16) + mt0) =
+            *reinterpret_cast<const uint32_t *>(gt + kDq8Rows * 128 + lane * 4);
+#pragma unroll
+    for (int u = 0; u < 2 * NJ; u++) {
+        const int r = 8 * u + (lane >> 3), ch = lane & 7;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(gt + r * 128 + ((ch ^ (r & 7)) << 4));
+        if (r < nr) *reinterpret_cast<u32x4 *>(A.dnh + (size_t)(c0 + r) * A.ldo + mt0 * 16 + ch * 8) = v;
+    }
+}
+
+// A tile's rows in chunks of at most 64, of as even a size as whole column
+// tiles allow (5 column tiles: 3 + 2).
+__device__ __forceinline__ void down_q8_tile(const GemmArgs &A, const uint8_t *W, int p0, int p1, int rb, uint8_t *sb,
+                                             float (*ssf)[kDlSfStride], float *ws, uint8_t *gt) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int mt0 = (rb * kDlW + wave) * kDlRT;
+    gt += wave * kDq8Gt;
+    const int nct = __builtin_amdgcn_readfirstlane((p1 - p0 + 15) >> 4);   // column tiles
+    const int nch = (nct + 3) >> 2, per = (nct + nch - 1) / nch;
+    for (int c0 = p0; c0 < p1; c0 += per * 16) {
+        const int nr = __builtin_amdgcn_readfirstlane(min(per * 16, p1 - c0));
+        if (c0 != p0) __syncthreads();   // previous chunk fully read
+        switch ((nr + 15) >> 4) {
+            case 1: down_q8_chunk<1>(A, W, mt0, c0, nr, sb, ssf, ws, gt); break;
+            case 2: down_q8_chunk<2>(A, W, mt0, c0, nr, sb, ssf, ws, gt); break;
+            case 3: down_q8_chunk<3>(A, W, mt0, c0, nr, sb, ssf, ws, gt); break;
+            default: down_q8_chunk<4>(A, W, mt0, c0, nr, sb, ssf, ws, gt); break;
         }
     }
 }
 
-// Q8: tiles whose down matrix is q8_0-split (routed: hq8, shared: shq8)
-// take down_q8_tile; the others, and every tile of an MXFP4 layer, the
-// body below.
-template <bool Q8>
-__global__ __launch_bounds__(64 * kDlW, Q8 ? 2 : 1) void k_down_lds(GemmArgs A) {
+// QM: which down matrices are q8_0-split (routed: hq8, shared: shq8): 0 none
+// (the body below for every tile), 2 all (down_q8_tile for every tile, in its
+// smaller LDS), 1 some.
+template <int QM>
+__global__ __launch_bounds__(64 * kDlW, QM ? 2 : 1) void k_down_lds(GemmArgs A) {
     constexpr int KD = 512, NKT = KD / 128, NRB = 2048 / (16 * kDlRT * kDlW);
-    __shared__ __align__(16) uint8_t sb[kDlRows * 512];
-    __shared__ uint32_t ss[kDlRows][4];       // B scale dwords: [row][lane group]
-    __shared__ float ws[kDlRows];             // routing weight of each row
-    __shared__ __align__(16) float ssf[Q8 ? kDlRows : 1][kDlSfStride];   // int8 h scales
+    // h rows of either body; the int8 body gathers its results behind its 64
+    constexpr int SB = QM == 2 ? kDq8Rows * 512 + kDlW * kDq8Gt : kDlRows * 512 + (QM ? kDlW * kDq8Gt - kDlRows * 256 : 0);
+    static_assert(kDq8Rows * 512 == kDlRows * 256, "the int8 rows take half of the MXFP4 rows' space");
+    constexpr int TS = QM == 2 ? 0 : kDlW * 16 * kDnT, SF = QM ? kDq8Rows * kDlSfStride * 4 : 0;
+    __shared__ __align__(16) uint8_t sb[SB];
+    __shared__ uint32_t ss[QM == 2 ? 1 : kDlRows][4];   // B scale dwords: [row][lane group]
+    __shared__ float ws[QM == 2 ? kDq8Rows : kDlRows];  // routing weight of each row
+    // the MXFP4 body's gathered rows or the int8 body's h scales
+    __shared__ __align__(16) uint8_t ts[TS > SF ? TS : SF];
     const int xcd = blockIdx.x & 7, jx = blockIdx.x >> 3;
     // tiles in reverse list order, as in k_gateup_dma
     const int ngrp = (*A.ntiles + 7) >> 3, grp = jx / NRB;
@@ -2156,12 +2226,14 @@ __global__ __launch_bounds__(64 * kDlW, Q8 ? 2 : 1) void k_down_lds(GemmArgs A) 
     if (ti >= *A.ntiles) return;
     const int4 tile = A.tiles[ti];
     const int e = __builtin_amdgcn_readfirstlane(tile.x), p0 = tile.y, p1 = tile.z;
-    if constexpr (Q8) {
-        if (e < A.E ? A.hq8 : A.shq8) {
-            down_q8_tile(A, e < A.E ? A.wa + (size_t)e * A.wstride : A.sa, p0, p1, rb, sb, ssf, ws);
+    if constexpr (QM) {
+        if (QM == 2 || (e < A.E ? A.hq8 : A.shq8)) {
+            down_q8_tile(A, e < A.E ? A.wa + (size_t)e * A.wstride : A.sa, p0, p1, rb, sb,
+                         reinterpret_cast<float (*)[kDlSfStride]>(ts), ws, sb + kDq8Rows * 512);
             return;
         }
     }
+    if constexpr (QM < 2) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, n = lane & 15;
     const uint8_t *W = e < A.E ? A.wa + (size_t)e * A.wstride : A.sa;
     const size_t nib = (size_t)2048 * KD / 2;
@@ -2210,8 +2282,10 @@ __global__ __launch_bounds__(64 * kDlW, Q8 ? 2 : 1) void k_down_lds(GemmArgs A) 
                     const v8i av = v8i{(int)f[0], (int)f[1], (int)f[2], (int)f[3], 0, 0, 0, 0};
                     acc[i] = mfma_sel(kt, av, bv[kt], acc[i], (int)sa[i], (int)sbw);
                 }
-            store_dn16x4(A, c0 + j * 16 + n, mt0, q, j * 16 + n < nr, acc, ws[r]);
+            store_dn16x4(A, nr - j * 16, mt0, q, n, acc, ws[r], ts + wave * 16 * kDnT,
+                         [&](int i) { return c0 + j * 16 + i; });
         }
+    }
     }
 }
 
@@ -2488,7 +2562,9 @@ __device__ __forceinline__ void skinny_expert(const GemmArgs &G, const GemmArgs 
         for (int j = 0; j < NJ; j++) {
             const int r = 16 * j + n;
             const v4f c4[4] = {acc[0][j], acc[1][j], acc[2][j], acc[3][j]};
-            store_dn16x4(Dn, L.ent[r], mt0, q, r < nr, c4, L.ws[r]);
+            // gathered in L.x, whose x rows every wave has read by now
+            store_dn16x4(Dn, nr - 16 * j, mt0, q, n, c4, L.ws[r], L.x + wave * 16 * kDnT,
+                         [&](int i) { return L.ent[16 * j + i]; });
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
         }
@@ -3884,11 +3960,14 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             break;
         case ST_DOWN:
             if (P.fused) break;   // in k_skinny_expert
-            if (P.da.hq8 || P.da.shq8)
-                hipLaunchKernelGGL(k_down_lds<true>, dim3(P.tiles * (D / (16 * kDlRT * kDlW))), dim3(64 * kDlW), 0, s,
+            if (P.da.hq8 && (P.da.shq8 || !P.has_sh))
+                hipLaunchKernelGGL(k_down_lds<2>, dim3(P.tiles * (D / (16 * kDlRT * kDlW))), dim3(64 * kDlW), 0, s,
+                                   P.da);
+            else if (P.da.hq8 || P.da.shq8)
+                hipLaunchKernelGGL(k_down_lds<1>, dim3(P.tiles * (D / (16 * kDlRT * kDlW))), dim3(64 * kDlW), 0, s,
                                    P.da);
             else
-                hipLaunchKernelGGL(k_down_lds<false>, dim3(P.tiles * (D / (16 * kDlRT * kDlW))), dim3(64 * kDlW), 0,
+                hipLaunchKernelGGL(k_down_lds<0>, dim3(P.tiles * (D / (16 * kDlRT * kDlW))), dim3(64 * kDlW), 0,
                                    s, P.da);
             break;
         case ST_COMBINE:

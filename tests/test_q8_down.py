@@ -682,6 +682,41 @@ def test_q8_shared_taps_and_replays(q8_shared_layer, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["mx", "both", "both, no shared", "mx, no shared"])
+def test_down_tile_sizes(q8_shared_layer, which):
+    """Fat tiles whose row counts sit on the edges of the down kernels' chunks
+    and column tiles (int8 and MXFP4 routed downs, with and without the int8
+    shared tiles beside them) against the direct path, which has no tiles."""
+    import torch
+    from q36_amd import moe
+    dw = q8_shared_layer[which.split(",")[0]]
+    T, E = 600, 256
+    g = torch.Generator(device="cuda").manual_seed(77)
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    rows = [1, 15, 16, 17, 31, 33, 47, 48, 63, 64, 65, 79, 80, 81, 127, 128, 129, 144, 145, 159, 160, 161, 321]
+    lg[:, :len(rows)] -= 100.0                # these experts are picked in their windows alone
+    at = 0
+    for e, r in enumerate(rows):
+        lg[(torch.arange(r, device="cuda") + at) % T, e] += 120.0
+        at += r
+    x = torch.randn(T, 2048, device="cuda", generator=g)
+    shg = None if "no shared" in which else torch.randn(T, device="cuda", generator=g)
+    layer = moe.MoELayer(T)
+    y = layer.forward(dw, x, lg, shg, out_dtype=torch.float32)
+    off = layer.tap(moe.TAP_EOFF)
+    assert layer.last_path == 0 and (off[1:] - off[:-1])[:len(rows)].tolist() == rows
+    ref = torch.cat([layer.forward(dw, x[t:t + 16], lg[t:t + 16], None if shg is None else shg[t:t + 16],
+                                   out_dtype=torch.float32) for t in range(0, T, 16)])
+    assert layer.last_path == 1
+    torch.cuda.synchronize()
+    # the 16-bit staging is 2^-11 of each term's group maximum, and h codes on
+    # rounding midpoints move by a step (2e-3, the module's bar, with room for
+    # a token's worst few)
+    err = (y - ref).abs().amax(1) / ref.abs().amax(1)
+    assert err.max() <= 5e-3 and err.median() <= 1e-3, (err.max(), err.median())
+
+
+@pytest.mark.gpu
 def test_q8_shared_refusals(q8_shared_layer):
     import torch
     from q36_amd import moe
