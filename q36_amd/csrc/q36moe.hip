@@ -23,8 +23,8 @@
 //              token order (q36_engine.cu:3393-3401).
 // q8_0-split matrices (the reference's requantised k-quant experts and its
 // Q8_0 shared expert) run on int8 MFMA with per-32 scales: down_q8_tile in
-// k_down_lds<1> and <2>, the Q8 branches of k_direct_down<true> and
-// k_direct_gateup<true, *>, and the shared gate/up body (k_shared_gateup_q8,
+// k_down_lds<1> and <2>, the Q8 branches of k_direct_down and
+// k_direct_gateup<2 or 8, *>, and the shared gate/up body (k_shared_gateup_q8,
 // or the leading workgroups of k_gateup_dma).  In front of the boundary:
 // k_router_f32 / k_router_f16 (router logits) and k_add_rmsnorm_quant (the
 // residual + RMSNorm + quantisation producer).
@@ -2932,8 +2932,14 @@ struct DirectGateupLds {
 // [512w, 512w+512) per 32 to int8 + fp32 scale into LDS and runs its 16
 // blocks against 16 rows of gate and up (int8 MFMA, each block scaled by
 // both scales); partial sums meet in LDS in wave order as in the MXFP4 body.
+// CH K-pairs of weights at a time, two such chunks in flight: all 8 at once
+// (128 registers) at the smallest batches, where one load latency counts; 2
+// from kDirectSh2 tokens, where those registers cost the routed workgroups of
+// the kernel their occupancy (3 waves per SIMD instead of 4).
+constexpr int kDirectSh2 = 3;
+template <int CH>
 __device__ __forceinline__ void direct_shared_q8(const DirectArgs &A, int t, int i, int ft, DirectGateupLds &L_) {
-    constexpr int NKP = kDD / 64, NKB = kDD / 32;
+    constexpr int NKP = kDD / 64, NKB = kDD / 32, NC = 8 / CH, NBUF = NC > 1 ? 2 : 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4;
     const bool col0 = (lane & 15) == 0;
@@ -2941,16 +2947,20 @@ __device__ __forceinline__ void direct_shared_q8(const DirectArgs &A, int t, int
     float *sxf = L_.sxf;
     const X8 xr = load8_raw(A.x, A.x_fmt, (size_t)t * kDD + wave * 512 + lane * 8);
     // this wave's 8 K-pairs of the gate and up row tile ft
-    u32x4 ag[8], au[8], sg[8], su[8];
+    struct Chunk { u32x4 ag[CH], au[CH], sg[CH], su[CH]; } w[NBUF];
+    auto load = [&](int c, Chunk &o) {
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const int kp = wave * 8 + u;
-        ag[u] = *reinterpret_cast<const u32x4 *>(A.sh_gate + ((size_t)ft * NKP + kp) * 1024 + lane * 16);
-        au[u] = *reinterpret_cast<const u32x4 *>(A.sh_up + ((size_t)ft * NKP + kp) * 1024 + lane * 16);
-        const size_t so = (size_t)kDF * kDD + (((size_t)ft * 4 + q) * NKB + 2 * kp) * 8;
-        sg[u] = *reinterpret_cast<const u32x4 *>(A.sh_gate + so);
-        su[u] = *reinterpret_cast<const u32x4 *>(A.sh_up + so);
-    }
+        for (int u = 0; u < CH; u++) {
+            const int kp = wave * 8 + c * CH + u;
+            o.ag[u] = *reinterpret_cast<const u32x4 *>(A.sh_gate + ((size_t)ft * NKP + kp) * 1024 + lane * 16);
+            o.au[u] = *reinterpret_cast<const u32x4 *>(A.sh_up + ((size_t)ft * NKP + kp) * 1024 + lane * 16);
+            const size_t so = (size_t)kDF * kDD + (((size_t)ft * 4 + q) * NKB + 2 * kp) * 8;
+            o.sg[u] = *reinterpret_cast<const u32x4 *>(A.sh_gate + so);
+            o.su[u] = *reinterpret_cast<const u32x4 *>(A.sh_up + so);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < NBUF; c++) load(c, w[c]);
     float v[8];
     cvt8(xr, A.x_fmt, v);
     float amax = 0.0f;
@@ -2965,33 +2975,38 @@ __device__ __forceinline__ void direct_shared_q8(const DirectArgs &A, int t, int
     __syncthreads();
     v4f cg = {0.f, 0.f, 0.f, 0.f}, cu = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 8; u++)
+    for (int c = 0; c < NC; c++) {
+        Chunk &o = w[c % NBUF];
+#pragma unroll
+        for (int u = 0; u < CH; u++)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int kb = 2 * (wave * 8 + u) + h;
+            const int kb = 2 * (wave * 8 + c * CH + u) + h;
             // column 0 is the token; lanes of other columns read zeros
             const uint2 bv = *reinterpret_cast<const uint2 *>(col0 ? sx + kb * 32 + 8 * q : sx + kDD);
             const long b = (long)(((uint64_t)bv.y << 32) | bv.x);
             const float dh = sxf[kb];
-            const long a0 = (long)(((uint64_t)ag[u][2 * h + 1] << 32) | ag[u][2 * h]);
-            const long a1 = (long)(((uint64_t)au[u][2 * h + 1] << 32) | au[u][2 * h]);
+            const long a0 = (long)(((uint64_t)o.ag[u][2 * h + 1] << 32) | o.ag[u][2 * h]);
+            const long a1 = (long)(((uint64_t)o.au[u][2 * h + 1] << 32) | o.au[u][2 * h]);
             const v4i bias = {kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias};
             const v4i gi = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, b, bias, 0, 0, 0);
             const v4i ui = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, b, bias, 0, 0, 0);
-            const uint32_t g01 = sg[u][2 * h], g23 = sg[u][2 * h + 1];
-            const uint32_t u01 = su[u][2 * h], u23 = su[u][2 * h + 1];
+            const uint32_t g01 = o.sg[u][2 * h], g23 = o.sg[u][2 * h + 1];
+            const uint32_t u01 = o.su[u][2 * h], u23 = o.su[u][2 * h + 1];
             const float wg[4] = {f16lo(g01), f16hi(g01), f16lo(g23), f16hi(g23)};
             const float wu[4] = {f16lo(u01), f16hi(u01), f16lo(u23), f16hi(u23)};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                cg[r] = fmaf(q8_scaled(gi[r], wg[r], -kQ8BiasF * wg[r]), dh, cg[r]);
-                cu[r] = fmaf(q8_scaled(ui[r], wu[r], -kQ8BiasF * wu[r]), dh, cu[r]);
+                cg[r] = fmaf(q8_scaled(gi[r], wg[r], q8_nwb(wg[r])), dh, cg[r]);
+                cu[r] = fmaf(q8_scaled(ui[r], wu[r], q8_nwb(wu[r])), dh, cu[r]);
             }
             // one block per scheduling group (otherwise all 32 MFMA results
             // are held at once)
             asm volatile("" : "+v"(cg), "+v"(cu));
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (c + NBUF < NC) load(c + NBUF, o);
+    }
     if (col0) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -3011,15 +3026,16 @@ __device__ __forceinline__ void direct_shared_q8(const DirectArgs &A, int t, int
 // weight loads in flight.  Measured (gate/up us, one tile / two): T=2 7.2 /
 // 7.5, T=4 9.8 / 10.0, T=8 16.5 / 15.5, T=16 27.4 / 25.6; four tiles at
 // T=16 25.7.
-template <bool SHQ8 = false, int NFT = 1, bool CACHED = false>
+// SHQ8: K-pairs per chunk of a q8_0-split shared expert's weights, 0 without one.
+template <int SHQ8 = 0, int NFT = 1, bool CACHED = false>
 __device__ __forceinline__ void direct_gateup_body(const DirectArgs &A, int i, int ft0,
                                                    DirectGateupLds &L_) {
     static_assert(NFT == 1 || NFT == 2, "row tiles per workgroup");
-    if constexpr (SHQ8) {   // workgroup-uniform: the shared expert's entries
+    if constexpr (SHQ8 != 0) {   // workgroup-uniform: the shared expert's entries
         const int nr0 = A.T * A.k;
         if (i >= nr0) {
 #pragma unroll
-            for (int u = 0; u < NFT; u++) direct_shared_q8(A, i - nr0, i, ft0 + u, L_);
+            for (int u = 0; u < NFT; u++) direct_shared_q8<SHQ8>(A, i - nr0, i, ft0 + u, L_);
             return;
         }
     }
@@ -3138,7 +3154,7 @@ __device__ __forceinline__ void direct_gateup_body(const DirectArgs &A, int i, i
     }
 }
 
-template <bool SHQ8, int NFT, bool CACHED = false>
+template <int SHQ8, int NFT, bool CACHED = false>
 __global__ __launch_bounds__(256) void k_direct_gateup(DirectArgs A) {
     __shared__ DirectGateupLds L_;
     direct_gateup_body<SHQ8, NFT, CACHED>(A, blockIdx.x, blockIdx.y * NFT, L_);
@@ -3151,8 +3167,16 @@ __global__ __launch_bounds__(256) void k_direct_gateup(DirectArgs A) {
 // matrix is q8_0-split (the routed slots with dn_q8, the shared expert with
 // sh_q8) quantise h per 32 to int8 with an fp32 scale (k_quant_q8b) and run
 // each 32-block as one int8 MFMA scaled by both scales (k_gemm_expert_i8).
-template <bool Q8, bool CACHED = false>
-__global__ __launch_bounds__(576) void k_direct_down(DirectArgs A) {
+// Q8: 0 no such matrix, 1 the shared expert's only, 2 and 3 any.  A wave's int8
+// tile is 64 registers at once; workgroups are 9 waves, so with the 112
+// registers that took, the kernel ran one per CU.  2 caps the kernel at 96
+// registers (two per CU), 1 takes the shared tile in halves (three per CU); 3,
+// below kDirectSh2 tokens, does neither: there every workgroup fits at once
+// and the cap or the second half's latency shows (1 token 10.2 -> 11.2 us).  Layer, us at T = 4 / 8 / 16, with the gate/up's chunks: Q8_0
+// shared 20.6 / 37.2 / 62.9 -> 19.0 / 34.2 / 55.3, int8 routed downs too 23.9
+// / 44.3 / 77.5 -> 23.1 / 40.4 / 72.7.
+template <int Q8, bool CACHED = false>
+__global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_down(DirectArgs A) {
     __shared__ __align__(16) uint8_t sh[kMaxTopK + 1][kDF + 32];
     __shared__ uint8_t shs[kMaxTopK + 1][kDF / 32];
     __shared__ float shf[Q8 ? kMaxTopK + 1 : 1][kDF / 32];
@@ -3162,7 +3186,8 @@ __global__ __launch_bounds__(576) void k_direct_down(DirectArgs A) {
     const int nslot = blockDim.x >> 6;
     const int nr = A.T * A.k;
     const bool routed = wave < A.k;
-    const bool wq8 = Q8 && (routed ? A.dn_q8 : A.sh_q8);   // wave-uniform: selects the MFMA kind
+    // wave-uniform: selects the MFMA kind
+    const bool wq8 = Q8 >= 2 ? (routed ? A.dn_q8 : A.sh_q8) : Q8 == 1 ? !routed : false;
     const int i = routed ? t * A.k + wave : nr + t;
     const int e = routed ? A.idx[i] : A.E;
     const float wgt = routed ? A.wt[i] : 1.0f / (1.0f + expf(-A.shg[(size_t)t * A.ld_shg]));
@@ -3172,17 +3197,18 @@ __global__ __launch_bounds__(576) void k_direct_down(DirectArgs A) {
     float hv[8];
     load8(A.hf, Q36MOE_FMT_F32, (size_t)i * kDF + lane * 8, hv);
     // phase 1: this wave's down tile into registers, its h row quantised into LDS
-    u32x4 ac[NKP], as[NKP];   // q8_0-split: codes and f16 scales
+    constexpr int NB = Q8 == 1 ? NKP / 2 : NKP;
+    u32x4 ac[NB], as[NB];     // q8_0-split: codes and f16 scales of NB K-pairs
     uint4 a[4];               // MXFP4: E2M1 fragments and the scale dword
     int sa = 0;
+    const uint8_t *Wq = routed ? A.down + (size_t)e * A.dn_wstride : A.sh_down;
+    auto load_q8 = [&](int kp) {
+        ac[kp % NB] = *reinterpret_cast<const u32x4 *>(Wq + ((size_t)rt * NKP + kp) * 1024 + lane * 16);
+        as[kp % NB] = *reinterpret_cast<const u32x4 *>(Wq + (size_t)kDD * kDF + (((size_t)rt * 4 + q) * NKB + 2 * kp) * 8);
+    };
     if (wq8) {
-        const uint8_t *W = routed ? A.down + (size_t)e * A.dn_wstride : A.sh_down;
-        const uint8_t *Wsc = W + (size_t)kDD * kDF;
 #pragma unroll
-        for (int kp = 0; kp < NKP; kp++) {
-            ac[kp] = *reinterpret_cast<const u32x4 *>(W + ((size_t)rt * NKP + kp) * 1024 + lane * 16);
-            as[kp] = *reinterpret_cast<const u32x4 *>(Wsc + (((size_t)rt * 4 + q) * NKB + 2 * kp) * 8);
-        }
+        for (int kp = 0; kp < NB; kp++) load_q8(kp);
         // lanes 4j..4j+3 hold block j
         float amax = 0.0f;
 #pragma unroll
@@ -3219,15 +3245,19 @@ __global__ __launch_bounds__(576) void k_direct_down(DirectArgs A) {
         for (int kb = 0; kb < NKB; kb++) {
             const uint2 bv = *reinterpret_cast<const uint2 *>(col0 ? &sh[wave][kb * 32 + 8 * q] : &sh[wave][kDF]);
             const long b = (long)(((uint64_t)bv.y << 32) | bv.x);
-            const u32x4 f = ac[kb >> 1];
+            const u32x4 f = ac[(kb >> 1) % NB];
             const long av = (kb & 1) ? (long)(((uint64_t)f[3] << 32) | f[2]) : (long)(((uint64_t)f[1] << 32) | f[0]);
             const v4i ci = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, b, v4i{kQ8Bias, kQ8Bias, kQ8Bias, kQ8Bias}, 0, 0, 0);
             const float dh = shf[wave][kb];
-            const u32x4 sv = as[kb >> 1];
+            const u32x4 sv = as[(kb >> 1) % NB];
             const uint32_t s01 = (kb & 1) ? sv[2] : sv[0], s23 = (kb & 1) ? sv[3] : sv[1];
             const float w[4] = {f16lo(s01), f16hi(s01), f16lo(s23), f16hi(s23)};
 #pragma unroll
-            for (int r = 0; r < 4; r++) c[r] = fmaf(q8_scaled(ci[r], w[r], -kQ8BiasF * w[r]), dh, c[r]);
+            for (int r = 0; r < 4; r++) c[r] = fmaf(q8_scaled(ci[r], w[r], q8_nwb(w[r])), dh, c[r]);
+            // one block per scheduling group, as in direct_shared_q8
+            asm volatile("" : "+v"(c));
+            __builtin_amdgcn_sched_barrier(0);
+            if ((kb & 1) && (kb >> 1) + NB < NKP) load_q8((kb >> 1) + NB);
         }
     } else {
         static_for<0, 4>([&](auto J) {
@@ -3908,27 +3938,33 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             static_assert(kDirectCachedT >= kDirect2Tiles, "cached loads only in the two-tile kernels");
             if (T >= kDirectCachedT) {
                 if (P.di.sh_q8)
-                    hipLaunchKernelGGL((k_direct_gateup<true, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
+                    hipLaunchKernelGGL((k_direct_gateup<2, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
                 else
-                    hipLaunchKernelGGL((k_direct_gateup<false, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
+                    hipLaunchKernelGGL((k_direct_gateup<0, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
             } else if (T >= kDirect2Tiles) {
                 if (P.di.sh_q8)
-                    hipLaunchKernelGGL((k_direct_gateup<true, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
+                    hipLaunchKernelGGL((k_direct_gateup<2, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
                 else
-                    hipLaunchKernelGGL((k_direct_gateup<false, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
+                    hipLaunchKernelGGL((k_direct_gateup<0, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
             } else {
-                if (P.di.sh_q8)
-                    hipLaunchKernelGGL((k_direct_gateup<true, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
+                if (P.di.sh_q8 && T >= kDirectSh2)
+                    hipLaunchKernelGGL((k_direct_gateup<2, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
+                else if (P.di.sh_q8)
+                    hipLaunchKernelGGL((k_direct_gateup<8, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
                 else
-                    hipLaunchKernelGGL((k_direct_gateup<false, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
+                    hipLaunchKernelGGL((k_direct_gateup<0, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
             }
         } else if (st == ST_DOWN) {
-            const bool q8 = P.di.dn_q8 || P.di.sh_q8, cached = T >= kDirectCachedT;
+            const int q8 = P.di.dn_q8 ? 2 : P.di.sh_q8 ? 1 : 0;
+            const bool cached = T >= kDirectCachedT;
             const dim3 g(D / 16, T), b(64 * (K + P.has_sh));
-            if (q8 && cached) hipLaunchKernelGGL((k_direct_down<true, true>), g, b, 0, s, P.di);
-            else if (q8) hipLaunchKernelGGL((k_direct_down<true, false>), g, b, 0, s, P.di);
-            else if (cached) hipLaunchKernelGGL((k_direct_down<false, true>), g, b, 0, s, P.di);
-            else hipLaunchKernelGGL((k_direct_down<false, false>), g, b, 0, s, P.di);
+            if (q8 && T < kDirectSh2) hipLaunchKernelGGL((k_direct_down<3, false>), g, b, 0, s, P.di);
+            else if (q8 == 2 && cached) hipLaunchKernelGGL((k_direct_down<2, true>), g, b, 0, s, P.di);
+            else if (q8 == 2) hipLaunchKernelGGL((k_direct_down<2, false>), g, b, 0, s, P.di);
+            else if (q8 && cached) hipLaunchKernelGGL((k_direct_down<1, true>), g, b, 0, s, P.di);
+            else if (q8) hipLaunchKernelGGL((k_direct_down<1, false>), g, b, 0, s, P.di);
+            else if (cached) hipLaunchKernelGGL((k_direct_down<0, true>), g, b, 0, s, P.di);
+            else hipLaunchKernelGGL((k_direct_down<0, false>), g, b, 0, s, P.di);
         }
         return;
     }

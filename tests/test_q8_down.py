@@ -647,9 +647,10 @@ def test_forward_q8_shared(oracle, q8_shared_layer, which, T, path):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("which", ["mx", "both"])
-@pytest.mark.parametrize("T", [17, 31, 33, 48, 130, 257, 512, 513])
+@pytest.mark.parametrize("T", [2, 3, 7, 8, 12, 16, 17, 31, 33, 48, 130, 257, 512, 513])
 def test_forward_q8_shared_small_batches(oracle, q8_shared_layer, which, T):
-    """The automatic path of small batches: the shared expert beside the
+    """The automatic path of small batches: the direct kernels' variants by
+    batch (2 and 3, 8, 12, 16 tokens), then the shared expert beside the
     routed tiles, at whole and partial tiles of 16 and 32 tokens, both row
     counts of the routed tiles and the path's limit (512 tokens)."""
     _check_shared_q8(oracle, q8_shared_layer, which, T, 0, 1500 + T)
