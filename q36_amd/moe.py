@@ -102,8 +102,14 @@ def check(rc, what):
 
 
 def _stream(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    """hipStream_t of `stream`, or of torch's current stream on the current
+    device, read without building a Stream object (2.9 -> 0.3 us, of the 12 us
+    that a one-kernel call such as router_logits takes on the host)."""
+    if stream is not None:
+        return stream.cuda_stream
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t, name, dtype=None):
@@ -113,7 +119,7 @@ def _dev(t, name, dtype=None):
         raise Q36MoEError(f"{name} must be contiguous")
     if dtype is not None and t.dtype != dtype:
         raise Q36MoEError(f"{name} must be {dtype}, got {t.dtype}")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _shg(shg, T):
@@ -130,7 +136,7 @@ def _shg(shg, T):
         raise Q36MoEError(f"shg must have T={T} elements, got {shg.shape[0]}")
     if T > 1 and shg.stride(0) < 1:
         raise Q36MoEError("shg must have a positive stride (no broadcast views)")
-    return ctypes.c_void_p(shg.data_ptr()), shg.stride(0) if T > 1 else 1
+    return shg.data_ptr(), shg.stride(0) if T > 1 else 1
 
 
 def _host_u8(a):
@@ -327,7 +333,7 @@ class MoELayer:
         ld = logits.stride(0)
         if logits.stride(1) != 1:
             raise Q36MoEError("logits rows must be contiguous")
-        lp = ctypes.c_void_p(logits.data_ptr()) if T else None
+        lp = logits.data_ptr() if T else None
         if T and (not logits.is_cuda or logits.dtype != torch.float32):
             raise Q36MoEError("logits must be a float32 GPU tensor")
         sp, sld = _shg(shg, T)
@@ -350,7 +356,7 @@ class MoELayer:
             raise Q36MoEError("logits must be [T, n_expert] with contiguous rows")
         if T and (not logits.is_cuda or logits.dtype != torch.float32):
             raise Q36MoEError("logits must be a float32 GPU tensor")
-        lp = ctypes.c_void_p(logits.data_ptr()) if T else None
+        lp = logits.data_ptr() if T else None
         sp, sld = _shg(shg, T)
         qp = _dev(xq, "xq", torch.uint8) if T else None
         sc = _dev(xs, "xs", torch.uint8) if T else None
@@ -377,7 +383,7 @@ class MoELayer:
         shape, dt = shapes[which]
         dst = torch.empty(shape, dtype=dt, device="cuda")
         n = ctypes.c_size_t()
-        check(lib().q36moe_ctx_copy_tap(self._h, which, ctypes.c_void_p(dst.data_ptr()),
+        check(lib().q36moe_ctx_copy_tap(self._h, which, dst.data_ptr(),
                                         dst.numel() * dst.element_size(), ctypes.byref(n)),
               "q36moe_ctx_copy_tap")
         return dst
@@ -446,11 +452,11 @@ def router_topk(logits, k=8, scale=1.0, renorm=True, n_expert=None):
     wt = torch.empty((T, k), dtype=torch.float32, device=logits.device)
     if logits.stride(1) != 1:
         raise Q36MoEError("logits rows must be contiguous")
-    lp = ctypes.c_void_p(logits.data_ptr()) if T else None
+    lp = logits.data_ptr() if T else None
     if T and (not logits.is_cuda or logits.dtype != torch.float32):
         raise Q36MoEError("logits must be a float32 GPU tensor")
     check(lib().q36moe_router_topk(lp, T, E, logits.stride(0), k, float(scale), 1 if renorm else 0,
-                                   ctypes.c_void_p(idx.data_ptr()), ctypes.c_void_p(wt.data_ptr()),
+                                   idx.data_ptr(), wt.data_ptr(),
                                    _stream()), "q36moe_router_topk")
     return idx, wt
 
@@ -471,8 +477,8 @@ def router_logits(w, x, n_expert, mode=ROUTER_AUTO):
     wp = _dev(w, "w", torch.float32)
     xp = _dev(x, "x") if T else None
     check(lib().q36moe_router_logits(wp, n_rows, n_expert, xp, fmt, T, x.shape[1], mode,
-                                     ctypes.c_void_p(logits.data_ptr()), n_expert,
-                                     ctypes.c_void_p(shg.data_ptr()) if shg is not None else None,
+                                     logits.data_ptr(), n_expert,
+                                     shg.data_ptr() if shg is not None else None,
                                      _stream()), "q36moe_router_logits")
     return logits, shg
 
@@ -540,7 +546,7 @@ def add_rmsnorm_quant(h, a, w, eps=1e-6, want_y=True, want_q=True):
     xs = torch.empty((T, D // 32), dtype=torch.uint8, device=h.device) if want_q else None
     hp = _dev(h, "h", torch.float32) if T else None
     ap = _dev(a, "a", torch.float32) if (a is not None and T) else None
-    ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if (t is not None and T) else None
+    ptr = lambda t: t.data_ptr() if (t is not None and T) else None
     check(lib().q36moe_add_rmsnorm_quant(hp, ap, _dev(w, "w", torch.float32), T, D, float(eps),
                                          ptr(y), ptr(xq), ptr(xs), _stream()), "q36moe_add_rmsnorm_quant")
     return y, xq, xs
@@ -554,8 +560,8 @@ def quant_e4m3(x):
     xs = torch.empty((T, K // 32), dtype=torch.uint8, device=x.device)
     fmt = FMT_F32 if x.dtype == torch.float32 else FMT_BF16
     xp = _dev(x, "x") if T else None
-    check(lib().q36moe_quant_e4m3(xp, fmt, T, K, ctypes.c_void_p(xq.data_ptr()),
-                                  ctypes.c_void_p(xs.data_ptr()), _stream()), "q36moe_quant_e4m3")
+    check(lib().q36moe_quant_e4m3(xp, fmt, T, K, xq.data_ptr(),
+                                  xs.data_ptr(), _stream()), "q36moe_quant_e4m3")
     return xq, xs
 
 
@@ -563,7 +569,7 @@ def probe_mfma(a, b, sa, sb, fmt_a, fmt_b):
     """One scaled 16x16x128 MFMA: a, b uint8 [64, 32]; sa, sb int32/uint32 [64]."""
     c = torch.empty((64, 4), dtype=torch.float32, device=a.device)
     check(lib().q36moe_probe_mfma(_dev(a, "a"), _dev(b, "b"), _dev(sa, "sa"), _dev(sb, "sb"),
-                                  fmt_a, fmt_b, ctypes.c_void_p(c.data_ptr()), _stream()),
+                                  fmt_a, fmt_b, c.data_ptr(), _stream()),
           "q36moe_probe_mfma")
     return c
 
@@ -573,7 +579,7 @@ def probe_mfma32(a, b, sa, sb):
     int32/uint32 [64] -> [64, 16] lane results."""
     c = torch.empty((64, 16), dtype=torch.float32, device=a.device)
     check(lib().q36moe_probe_mfma32(_dev(a, "a"), _dev(b, "b"), _dev(sa, "sa"), _dev(sb, "sb"),
-                                    ctypes.c_void_p(c.data_ptr()), _stream()), "q36moe_probe_mfma32")
+                                    c.data_ptr(), _stream()), "q36moe_probe_mfma32")
     return c
 
 
@@ -598,7 +604,7 @@ def forward_noalloc(weights, x, logits, shg=None, top_k=8, scale=1.0, out=None, 
         raise Q36MoEError("logits must be a float32 GPU tensor")
     sp, sld = _shg(shg, T)
     check(lib().q36moe_forward_noalloc(weights._h, _dev(x, "x") if T else None, xf,
-                                       ctypes.c_void_p(logits.data_ptr()) if T else None, logits.stride(0),
+                                       logits.data_ptr() if T else None, logits.stride(0),
                                        sp, sld, T, top_k, float(scale), _dev(out, "out") if T else None, of,
                                        _stream(stream)), "q36moe_forward_noalloc")
     return out
