@@ -24,7 +24,7 @@
 // q8_0-split matrices (the reference's requantised k-quant experts and its
 // Q8_0 shared expert) run on int8 MFMA with per-32 scales: down_q8_tile in
 // k_down_lds<1> and <2>, the Q8 branches of k_direct_down and
-// k_direct_gateup<2 or 8, *>, and the shared gate/up body (k_shared_gateup_q8,
+// k_direct_gateup<2 or 8, *>, and the shared gate/up bodies (sh8_gateup and,
 // or the leading workgroups of k_gateup_dma).  In front of the boundary:
 // k_router_f32 / k_router_f16 (router logits) and k_add_rmsnorm_quant (the
 // residual + RMSNorm + quantisation producer).
@@ -1012,7 +1012,8 @@ struct GemmArgs {
     int hq8;
     float *hsf; const float *bsf;
     // q8_0-split shared expert: its tiles are skipped by the MXFP4 gate/up
-    // kernels (k_shared_gateup_q8 computes its rows from the int8 x) and run
+    // kernels (sh8_gateup or shared_gateup_q8_body computes its rows from the
+    // int8 x) and run
     // down_q8_tile in DOWN
     int shq8;
     const int8_t *xq8; const float *xsf;   // int8 x [T][K] + fp32 scales [T][K/32]
@@ -1505,13 +1506,6 @@ __device__ __forceinline__ void shared_gateup_q8_body(const GemmArgs &A, int tb,
     }
 }
 
-// Stand-alone launch (skinny-tile layers); fat-tile layers run the same
-// body in k_gateup_dma's first workgroups, beside the routed tiles.
-__global__ __launch_bounds__(256, 2) void k_shared_gateup_q8(GemmArgs A) {
-    __shared__ __align__(16) uint8_t lds[kShLds];
-    shared_gateup_q8_body(A, blockIdx.x, blockIdx.y, lds);
-}
-
 __global__ __launch_bounds__(256, 2) void k_gateup_dma(GemmArgs A) {
     __shared__ gdma::Lds L;
     constexpr int NRB = 512 / (16 * gdma::RT);
@@ -1538,7 +1532,7 @@ __global__ __launch_bounds__(256, 2) void k_gateup_dma(GemmArgs A) {
     if (ti >= *A.ntiles) return;
     const int4 tile = A.tiles[ti];
     const int e = tile.x, p0 = tile.y, p1 = tile.z;
-    if (e == A.E && A.shq8) return;      // k_shared_gateup_q8's rows
+    if (e == A.E && A.shq8) return;      // rows of the int8 shared gate/up
     const uint8_t *Wg = e < A.E ? A.wa + (size_t)e * A.wstride : A.sa;
     const uint8_t *Wu = e < A.E ? A.wb + (size_t)e * A.wstride : A.sb;
     const int ntt = (p1 - p0 + 15) >> 4;
@@ -1990,7 +1984,7 @@ __global__ __launch_bounds__(64 * kSkW) void k_skinny_gateup(GemmArgs A) {
     const int nj = (p1 - p0 + 15) >> 4;
     const uint8_t *Wg = e < A.E ? A.wa + (size_t)e * A.wstride : A.sa;
     const uint8_t *Wu = e < A.E ? A.wb + (size_t)e * A.wstride : A.sb;
-    if (e == A.E && A.shq8) return;      // k_shared_gateup_q8's rows
+    if (e == A.E && A.shq8) return;      // rows of the int8 shared gate/up
     const bool hq8 = A.hq8 && e < A.E;   // shared rows: an MXFP4 down
     if (nj <= 1) skinny_gateup<1>(A, Wg, Wu, rb * 2, p0, p1, red, hq8);
     else skinny_gateup<2>(A, Wg, Wu, rb * 2, p0, p1, red, hq8);
@@ -2878,6 +2872,15 @@ __device__ __forceinline__ void sh8_gateup(const GemmArgs &A, SxLds &L, int tb, 
         for (int i = 0; i < 4; i++) h[r][i] = silu(sum[r][i]) * sum[2 + r][i];
     const int t = t0 + 16 * wave + n;
     store_h_block(A, true, A.nrouted + t, t < A.T, mt0 * 16, q, lane, h);
+}
+
+// The same for layers whose tiles run as separate gate/up and down kernels (an
+// int8 routed down).  Layer, us at T = 17 / 48 / 128 / 256: 127 / 168 / 191 / 200
+// with the 256-token workgroups of the fat tiles' shared body as this launch (16
+// workgroups, 61 us); 78 / 115 / 135 / 145 this way.
+__global__ __launch_bounds__(64 * kSxW) void k_sh8_gateup(GemmArgs A) {
+    __shared__ SxLds L;
+    sh8_gateup(A, L, blockIdx.x / kShRb, blockIdx.x % kShRb);
 }
 
 // SH8: with the extra workgroups of a q8_0-split shared expert (a template
@@ -4042,7 +4045,7 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             } else if (P.skinny) {
                 hipLaunchKernelGGL(k_skinny_gateup, dim3(P.tiles * 16), dim3(64 * kSkW), 0, s, P.ga);
                 if (P.ga.shq8)
-                    hipLaunchKernelGGL(k_shared_gateup_q8, dim3((T + kShTok - 1) / kShTok, kShRb), dim3(256), 0, s,
+                    hipLaunchKernelGGL(k_sh8_gateup, dim3((T + kSh8Tok - 1) / kSh8Tok * kShRb), dim3(64 * kSxW), 0, s,
                                        P.ga);
             } else
                 hipLaunchKernelGGL(k_gateup_dma, dim3(P.tiles * (FF / (16 * gdma::RT)) + P.ga.sh_wgs),
