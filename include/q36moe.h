@@ -244,7 +244,9 @@ int q36moe_forward_q8(q36moe_ctx *c, const q36moe_weights *w, const uint8_t *xq,
  * slots combined in registers) serves T <= 16 as two kernels (gate/up, then
  * down).  Skinny tiles run either as one kernel per tile (gate/up, h kept
  * in LDS, down) or as separate gate/up and down kernels; the one-kernel
- * form needs MXFP4 down and shared-expert matrices.  mode 0 picks the
+ * form needs an MXFP4 routed down, and an MXFP4 shared expert unless the path
+ * is chosen automatically and T*k <= 4096 (a q8_0-split shared expert then
+ * runs beside the routed tiles and in the combine).  mode 0 picks the
  * direct path for T <= 16, skinny tiles (one kernel per tile where it
  * applies) while T*k <= 8*n_expert (16*n_expert when the one-kernel form
  * applies) and fat tiles above; 1 forces sorted with

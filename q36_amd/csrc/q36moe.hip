@@ -24,8 +24,9 @@
 // q8_0-split matrices (the reference's requantised k-quant experts and its
 // Q8_0 shared expert) run on int8 MFMA with per-32 scales: down_q8_tile in
 // k_down_lds<1> and <2>, the Q8 branches of k_direct_down and
-// k_direct_gateup<2 or 8, *>, and the shared gate/up bodies (sh8_gateup and,
-// or the leading workgroups of k_gateup_dma).  In front of the boundary:
+// k_direct_gateup<2 or 8, *>, and the shared gate/up bodies (sh8_gateup for
+// small batches, shared_gateup_q8_body in the leading workgroups of
+// k_gateup_dma).  In front of the boundary:
 // k_router_f32 / k_router_f16 (router logits) and k_add_rmsnorm_quant (the
 // residual + RMSNorm + quantisation producer).
 #include <hip/hip_runtime.h>

@@ -771,3 +771,36 @@ def test_q8_layer_in_hip_graph(q8_shared_layer, T):
         other = layer.forward(dw, x2, lg2, shg, out_dtype=torch.float32)
         torch.cuda.synchronize()
         assert not torch.equal(other, ref)
+
+
+@pytest.mark.gpu
+def test_q8_shared_beside_tiles_in_hip_graph(q8_shared_layer):
+    """The shared expert beside the routed tiles (40 tokens) under capture:
+    replays with eager work and synchronisations between give the eager bits."""
+    import torch
+    from q36_amd import moe
+    dw, T = q8_shared_layer["mx"], 40
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, x2 = (torch.randn(T, 2048, device="cuda", generator=g) for _ in range(2))
+    lg, lg2 = (torch.randn(T, 256, device="cuda", generator=g) for _ in range(2))
+    shg = torch.randn(T, device="cuda", generator=g)
+    layer = moe.MoELayer(T)
+    out = torch.empty((T, 2048), dtype=torch.float32, device="cuda")
+    ref = layer.forward(dw, x, lg, shg, out_dtype=torch.float32).clone()
+    assert layer.last_path == 3
+    cap = torch.cuda.Stream()
+    layer.set_stream(cap)
+    torch.cuda.synchronize()
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr, stream=cap):
+        layer.forward(dw, x, lg, shg, out=out)
+    torch.cuda.synchronize()
+    layer.set_stream(torch.cuda.current_stream())
+    for rep in range(3):
+        out.zero_()
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), f"replay {rep}"
+        other = layer.forward(dw, x2, lg2, shg, out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        assert not torch.equal(other, ref)
