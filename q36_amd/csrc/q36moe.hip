@@ -2009,8 +2009,8 @@ constexpr int kDlRows = 128;             // B rows staged per chunk
 // Staging of a weighted down row: f16 with a power-of-two scale per 16
 // columns.  The 16 columns of group g of row p are held by lanes q = 0..3 of
 // one MFMA column, 4 each; their maximum |v| has the biased fp32 exponent eb
-// (clamped to [15, 254]; 255 keeps inf / NaN), the group is stored as
-// v * 2^(141 - eb) (exact: a power of two), every value of which is below
+// (at least 15, and see dn16_scale; 255 keeps inf / NaN), the group is stored
+// as v * 2^(141 - eb) (exact: a power of two), every value of which is below
 // 2^15 < 65504, rounded to f16 (RNE, relative error <= 2^-11), with eb in
 // dne; the combine multiplies back by 2^(eb - 141).  Half the bytes of an
 // f32 staging (which the reference uses, q36_engine.cu:3451-3463) for a
@@ -2021,10 +2021,15 @@ __device__ __forceinline__ uint2 dn16_pack(float v0, float v1, float v2, float v
     const f16x2v lo = __builtin_convertvector((f32x2){v0, v1}, f16x2v), hi = __builtin_convertvector((f32x2){v2, v3}, f16x2v);
     return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
 }
-// v * 2^(141 - eb) times the routing weight w for a group whose maximum |v| * |w|
-// is a: the multiplier (w folded into the power of two, exact) and eb.
+// The multiplier w * 2^(141 - eb) of a group of unweighted results c with
+// routing weight w and a = max |c| * |w|, and eb.  eb is at least w's biased
+// exponent - 113, so the product, at most 2^128 - 2^104 then, stays finite for
+// every finite w: an all-zero group (x = 0) of a weight of 4 or more, with
+// eb = 15, would be 0 * inf.  A normal c of a group that this raises is still
+// stored at 2 or above, with all of f16's bits.
 __device__ __forceinline__ float dn16_scale(float a, float w, uint32_t &eb) {
-    eb = max((__float_as_uint(a) >> 23) & 0xffu, 15u);
+    const uint32_t ew = (__float_as_uint(w) >> 23) & 0xffu;
+    eb = max((__float_as_uint(a) >> 23) & 0xffu, max(ew, 128u) - 113u);
     return w * __uint_as_float((268u - eb) << 23);
 }
 

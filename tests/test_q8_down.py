@@ -718,6 +718,41 @@ def test_down_tile_sizes(q8_shared_layer, which):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scale", [8.0, 2.0 ** 100])
+@pytest.mark.parametrize("k", [8, 1])
+@pytest.mark.parametrize("which,path", [("mxfp4", 1), ("mxfp4", 4), ("mxfp4", 5), ("mx", 0), ("mx", 1), ("mx", 4),
+                                        ("both", 1), ("both", 4)])
+def test_zero_rows_of_large_weights(q8_shared_layer, which, path, k, scale):
+    """Tokens with x = 0 give exactly 0 whatever the routing weight: the staged
+    rows' power of two, with the weight folded in, stays finite for an all-zero
+    group.  The other tokens against the direct path, which stages nothing."""
+    import torch
+    from q36_amd import moe
+    T, E = 70, 256
+    dw = moe.MoEWeights.alloc(E, 2048, 512, 512).fill_synthetic(11, -9, -5) if which == "mxfp4" else q8_shared_layer[which]
+    g = torch.Generator(device="cuda").manual_seed(100 * k + path)
+    x = torch.randn(T, 2048, device="cuda", generator=g)
+    x[::3] = 0.0
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    shg = torch.randn(T, device="cuda", generator=g)
+    layer = moe.MoELayer(T, top_k=k)
+    layer.set_path(path)
+    y = layer.forward(dw, x, lg, shg, scale=scale, out_dtype=torch.float32)
+    assert layer.last_path == {0: 3, 1: 0, 4: 2, 5: 3}[path]
+    layer.set_path(layer.PATH_DIRECT)
+    ref = torch.cat([layer.forward(dw, x[t:t + 16], lg[t:t + 16], shg[t:t + 16], scale=scale, out_dtype=torch.float32)
+                     for t in range(0, T, 16)])
+    torch.cuda.synchronize()
+    zero = torch.arange(T, device="cuda") % 3 == 0
+    assert (ref[zero] == 0).all() and torch.isfinite(ref).all()
+    assert (y[zero] == 0).all(), y[zero].isnan().sum()
+    # the bars of test_down_tile_sizes, in fp64 (2^100 squared leaves fp32)
+    y, ref = y[~zero].double(), ref[~zero].double()
+    err = (y - ref).abs().amax(1) / ref.abs().amax(1)
+    assert err.max() <= 5e-3 and err.median() <= 1e-3, (err.max(), err.median())
+
+
+@pytest.mark.gpu
 def test_q8_shared_refusals(q8_shared_layer):
     import torch
     from q36_amd import moe
