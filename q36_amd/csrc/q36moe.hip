@@ -1570,31 +1570,42 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// Workgroup = one router row, wave w = NT tokens (w, w + waves, ...): the
-// tokens' dot products run side by side, where one wave walking the tokens
-// paid an L2 round trip for each.  At most kRfW waves, so that a wave's row
-// and tokens are all in flight at once (16 waves leave 64 registers each,
-// which a row and a token fill).  Same products and order of sums whatever T.
-// us at T = 1 / 4 / 7 / 16, 257 rows: 2.4 / 3.6 / 4.9 / 8.7 with one wave per
-// row walking the tokens, 2.5 / 2.8 / 3.4 / 4.9 now (1: a launch's floor).
+// Workgroup = one router row.  With few rows a wave takes NT tokens (w,
+// w + waves, ...), so the tokens' dot products run side by side where one wave
+// walking the tokens pays an L2 round trip for each: up to kRfW tokens a wave
+// per token (NW = 0: no loop and no count of waves to read), beyond that NW =
+// kRfW waves of two tokens, so that a wave's row and tokens are all in flight
+// at once (16 waves leave 64 registers each, which a row and a token fill).
+// With many rows, whose waves fill the chip and share the L1's bandwidth, one
+// wave walks the tokens with its row in registers (from some 3000 rows on, when
+// enough waves share a CU to cover a load, without PIN: 16 tokens and 1025 /
+// 2049 / 4097 rows 8.6 / 10.4 / 21.0 us with it, 10.1 / 11.3 / 18.7 without).
+// Same products and order of sums whatever T.  us at T = 1 / 4 / 7 / 9 / 16, one wave per row against the
+// waves per token (launch_router's limits):
+//    257 rows   2.4 / 3.5 / 5.0 /  5.4 /  8.1    2.4 / 2.7 / 3.5 /  4.6 /  4.7
+//    513        2.5 / 3.6 / 5.1 /  5.5 /  8.3    2.5 / 3.1 / 4.3 /  5.9 /  6.1
+//    769        2.5 / 3.7 / 5.2 /  5.6 /  8.4    2.5 / 3.5 / 5.2 /  7.2 /  7.5
+//   1025        2.6 / 3.9 / 5.4 /  5.8 /  8.6    2.6 / 3.9 / 6.1 /  8.5 /  8.8
+//   4097        4.2 / 7.3 /11.7 / 12.8 / 21      4.2 / 9.8 /17.3 / 25   / 26.5
 constexpr int kRfW = 8;
-template <int XF, int NT>
-__global__ __launch_bounds__(64 * kRfW) void k_router_f32(const float *__restrict__ W, int n_expert,
-                                                         const void *__restrict__ x, int T,
-                                                         float *__restrict__ logits, int ld,
-                                                         float *__restrict__ shg) {
+template <int XF, int NT, int NW, bool PIN = true>
+__global__ __launch_bounds__(64 * (NW ? NW : kRfW)) void k_router_f32(const float *__restrict__ W, int n_expert,
+                                                                     const void *__restrict__ x, int T,
+                                                                     float *__restrict__ logits, int ld,
+                                                                     float *__restrict__ shg) {
+    static_assert(NW || NT == 1, "a wave per token");
     const int r = blockIdx.x, lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float *w = W + (size_t)r * kRtD;
     float4 wv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) wv[j] = *reinterpret_cast<const float4 *>(w + (j * 64 + lane) * 4);
-    for (int t0 = wave; t0 < T; t0 += nw * NT) {
+    for (int t0 = wave; NW == 0 || t0 < T; t0 += NW * NT) {
         u32x4 xf[NT][8];   // fp32 x
         uint2 xh[NT][8];   // bf16 x
 #pragma unroll
         for (int u = 0; u < NT; u++) {
-            const size_t o = (size_t)min(t0 + u * nw, T - 1) * kRtD;   // past the end: the last token again, not stored
+            const size_t o = (size_t)min(t0 + u * NW, T - 1) * kRtD;   // past the end: the last token again, not stored
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 if constexpr (XF == Q36MOE_FMT_F32)
@@ -1605,7 +1616,7 @@ __global__ __launch_bounds__(64 * kRfW) void k_router_f32(const float *__restric
         }
         // every load issued before the first product: left alone, the compiler
         // keeps four of a token's eight in flight
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < NT; u++) {
             float acc = 0.0f;
@@ -1625,12 +1636,13 @@ __global__ __launch_bounds__(64 * kRfW) void k_router_f32(const float *__restric
                 acc = fmaf(wv[j].w, xv[3], acc);
             }
             acc = wave_sum(acc);
-            const int t = t0 + u * nw;
+            const int t = t0 + u * NW;
             if (lane == 0 && t < T) {
                 if (r < n_expert) logits[(size_t)t * ld + r] = acc;
                 else shg[t] = acc;
             }
         }
+        if constexpr (NW == 0) break;
     }
 }
 
@@ -1813,10 +1825,16 @@ template <int XF>
 static void launch_router(bool f16, const float *w, int n_rows, int n_expert, const void *x, int T, float *logits,
                           int ld, float *shg, hipStream_t s) {
     if (!f16) {
-        if (T <= kRfW)
-            hipLaunchKernelGGL((k_router_f32<XF, 1>), dim3(n_rows), dim3(64 * T), 0, s, w, n_expert, x, T, logits, ld, shg);
+        if (T == 1 || (T <= kRfW && n_rows <= 768))
+            hipLaunchKernelGGL((k_router_f32<XF, 1, 0>), dim3(n_rows), dim3(64 * T), 0, s, w, n_expert, x, T, logits, ld, shg);
+        else if (T > kRfW && n_rows <= 512)
+            hipLaunchKernelGGL((k_router_f32<XF, 2, kRfW>), dim3(n_rows), dim3(64 * kRfW), 0, s, w, n_expert, x, T, logits, ld,
+                               shg);
+        else if (n_rows <= 3072)
+            hipLaunchKernelGGL((k_router_f32<XF, 1, 1>), dim3(n_rows), dim3(64), 0, s, w, n_expert, x, T, logits, ld, shg);
         else
-            hipLaunchKernelGGL((k_router_f32<XF, 2>), dim3(n_rows), dim3(64 * kRfW), 0, s, w, n_expert, x, T, logits, ld, shg);
+            hipLaunchKernelGGL((k_router_f32<XF, 1, 1, false>), dim3(n_rows), dim3(64), 0, s, w, n_expert, x, T, logits, ld,
+                               shg);
         return;
     }
     const int nrb1 = (n_rows + 15) / 16, nrb2 = (n_rows + 31) / 32;
