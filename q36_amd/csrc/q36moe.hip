@@ -3248,14 +3248,15 @@ __global__ __launch_bounds__(256) void k_direct_gateup(DirectArgs A) {
 // matrix is q8_0-split (the routed slots with dn_q8, the shared expert with
 // sh_q8) quantise h per 32 to int8 with an fp32 scale (k_quant_q8b) and run
 // each 32-block as one int8 MFMA scaled by both scales (k_gemm_expert_i8).
-// Q8: 0 no such matrix, 1 the shared expert's only, 2 and 3 any.  A wave's int8
+// Q8: 0 no such matrix, 1 the shared expert's only, 2 any.  A wave's int8
 // tile is 64 registers at once; workgroups are 9 waves, so with the 112
-// registers that took, the kernel ran one per CU.  2 caps the kernel at 96
-// registers (two per CU), 1 takes the shared tile in halves (three per CU); 3,
-// below kDirectSh2 tokens, does neither: there every workgroup fits at once
-// and the cap or the second half's latency shows (1 token 10.2 -> 11.2 us).  Layer, us at T = 4 / 8 / 16, with the gate/up's chunks: Q8_0
-// shared 20.6 / 37.2 / 62.9 -> 19.0 / 34.2 / 55.3, int8 routed downs too 23.9
-// / 44.3 / 77.5 -> 23.1 / 40.4 / 72.7.
+// registers that took, the kernel ran one per CU.  2 fits in 96 registers (two
+// per CU), 1 takes the shared tile in halves and fits in 72 (three per CU);
+// below kDirectSh2 tokens every workgroup fits at once and the second half's
+// latency shows (1 token 10.2 -> 11.2 us), so 2 serves both.  Layer, us at T =
+// 4 / 8 / 16, with the gate/up's chunks: Q8_0 shared 20.9 / 37.2 / 59.2 -> 18.0
+// / 32.1 / 49.4, int8 routed downs too 24.2 / 43.5 / 74.4 -> 22.8 / 40.0 / 67.7
+// (of that 1.0 / 2.4 / 3.7 and 0.7 / 0.9 / 2.4 from the spills, see ac).
 template <int Q8, bool CACHED = false>
 __global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_down(DirectArgs A) {
     __shared__ __align__(16) uint8_t sh[kMaxTopK + 1][kDF + 32];
@@ -3279,8 +3280,12 @@ __global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_d
     load8(A.hf, Q36MOE_FMT_F32, (size_t)i * kDF + lane * 8, hv);
     // phase 1: this wave's down tile into registers, its h row quantised into LDS
     constexpr int NB = Q8 == 1 ? NKP / 2 : NKP;
-    u32x4 ac[NB], as[NB];     // q8_0-split: codes and f16 scales of NB K-pairs
-    uint4 a[4];               // MXFP4: E2M1 fragments and the scale dword
+    // the wave's down tile.  q8_0-split: codes and f16 scales of NB K-pairs;
+    // MXFP4: its 4 E2M1 fragments in ac and the scale dword sa (in registers of
+    // their own they stayed live beside ac over the barrier that both kinds
+    // share, which at the caps spilled 8 registers to scratch memory)
+    static_assert(NB >= 4, "4 MXFP4 fragments");
+    u32x4 ac[NB], as[NB];
     int sa = 0;
     const uint8_t *Wq = routed ? A.down + (size_t)e * A.dn_wstride : A.sh_down;
     auto load_q8 = [&](int kp) {
@@ -3308,7 +3313,7 @@ __global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_d
         const size_t nib = (size_t)kDD * kDF / 2;
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            { const u32x4 t = direct_ld16<CACHED>(W + ((size_t)rt * 4 + j) * 1024 + (size_t)lane * 16); a[j] = make_uint4(t[0], t[1], t[2], t[3]); }
+            ac[j] = direct_ld16<CACHED>(W + ((size_t)rt * 4 + j) * 1024 + (size_t)lane * 16);
         sa = *reinterpret_cast<const int *>(W + nib + ((size_t)rt * 64 + lane) * 4);
         quant8_lane(hv, lane, &sh[wave][lane * 8], &shs[wave][lane >> 2]);
         if (rt == 0) {   // quantised h (tap)
@@ -3350,7 +3355,7 @@ __global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_d
             const v8i b = v8i{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w,
                               (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
             const int sb = shs[wave][j * 4 + q];
-            const v8i av = v8i{(int)a[j].x, (int)a[j].y, (int)a[j].z, (int)a[j].w, 0, 0, 0, 0};
+            const v8i av = v8i{(int)ac[j][0], (int)ac[j][1], (int)ac[j][2], (int)ac[j][3], 0, 0, 0, 0};
             c = mfma_f4xf8<j>(av, b, c, sa, sb);
         });
     }
@@ -4039,7 +4044,7 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             const int q8 = P.di.dn_q8 ? 2 : P.di.sh_q8 ? 1 : 0;
             const bool cached = T >= kDirectCachedT;
             const dim3 g(D / 16, T), b(64 * (K + P.has_sh));
-            if (q8 && T < kDirectSh2) hipLaunchKernelGGL((k_direct_down<3, false>), g, b, 0, s, P.di);
+            if (q8 && T < kDirectSh2) hipLaunchKernelGGL((k_direct_down<2, false>), g, b, 0, s, P.di);
             else if (q8 == 2 && cached) hipLaunchKernelGGL((k_direct_down<2, true>), g, b, 0, s, P.di);
             else if (q8 == 2) hipLaunchKernelGGL((k_direct_down<2, false>), g, b, 0, s, P.di);
             else if (q8 && cached) hipLaunchKernelGGL((k_direct_down<1, true>), g, b, 0, s, P.di);
