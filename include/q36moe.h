@@ -245,8 +245,9 @@ int q36moe_forward_q8(q36moe_ctx *c, const q36moe_weights *w, const uint8_t *xq,
  * down).  Skinny tiles run either as one kernel per tile (gate/up, h kept
  * in LDS, down) or as separate gate/up and down kernels; the one-kernel
  * form needs an MXFP4 routed down, and an MXFP4 shared expert unless the path
- * is chosen automatically and T*k <= 4096 (a q8_0-split shared expert then
- * runs beside the routed tiles and in the combine).  mode 0 picks the
+ * is chosen automatically, T*k <= 4096 and T <= 1280 (a q8_0-split shared
+ * expert then runs beside the routed tiles and in the combine; above 1280
+ * tokens such a layer takes fat tiles).  mode 0 picks the
  * direct path for T <= 16, skinny tiles (one kernel per tile where it
  * applies) while T*k <= 8*n_expert (16*n_expert when the one-kernel form
  * applies) and fat tiles above; 1 forces sorted with

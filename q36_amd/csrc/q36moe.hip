@@ -2797,7 +2797,13 @@ __device__ __forceinline__ void sx_gather(const SxArgs &X, SxLds &L, int e, int 
 // experts: 115 / 136 / 166 / 177 / 122 with separate gate/up, shared gate/up
 // (61 us in 16 workgroups) and down kernels, or fat tiles from T = 257;
 // 50 / 58 / 83 / 87 / 109 this way.
+// Every 32 tokens read their share of the 2 MiB of weights again, so at a small
+// top_k, where many tokens have few routed rows, fat tiles with 256 tokens per
+// shared workgroup win from about 1250 tokens on (top_k 1, T = 1000 / 1250 /
+// 1500 / 2048 / 4096: 103 / 113 / 117 / 132 / 201 against 110 / 113 / 116 / 128
+// / 162 us; the same crossing at top_k 2 and 3).
 constexpr int kSh8Tok = 32;              // tokens per workgroup (two column tiles)
+constexpr int kSh8MaxT = 1280;           // auto mode: most tokens of this form beside MXFP4 tiles
 constexpr int kSh8Sf = 66;               // floats per staged row of x scales
 static_assert(kSh8Tok == kSkTok && sizeof(float) * kSh8Tok * kSh8Sf <= sizeof(SxLds::h), "x and its scales fit L.x / L.h");
 static_assert(kSxW * 4 * (kSh8Tok / 16) * 64 * 16 <= sizeof(SxLds::x), "the partial sums fit L.x");
@@ -4155,16 +4161,18 @@ static int launch_forward(const Scratch &c, Plan &P, int pm, const q36moe_weight
     if (shq8 && x_fmt == kFmtE4M3) return Q36MOE_EINVAL;
     // sorted path: skinny tiles (<= 32 rows) while the average expert has at
     // most kSkinnyRows rows, else fat tiles of up to kGdTok rows
-    // the one-kernel skinny path (every matrix MXFP4) serves twice the rows
+    // the one-kernel skinny path (routed experts MXFP4) serves twice the rows
     // per expert: it beat fat tiles up to 512 tokens (T=384: 96 vs 103 us)
     // a q8_0-split shared expert rides along (its gate/up in extra workgroups
     // of that launch, its down in the combine) where the tiles are found
-    // in-kernel; a forced path keeps the two kernels
+    // in-kernel; a forced path keeps the two kernels, and above kSh8MaxT tokens
+    // fat tiles take over whatever T*k
+    const bool many_sh8 = shq8 && !w->dn_q8 && T > kSh8MaxT;
     const bool fusable = !w->dn_q8 && (!shq8 || (pm == 0 && n <= kSxDiscoverMax));
     const size_t skinny_rows = (size_t)(fusable ? kSxFusedRows : kSkinnyRows) * E;
-    const bool skinny = pm == 4 || pm == 5 || (pm == 0 && (size_t)n <= skinny_rows);
-    // skinny tiles in one kernel per tile (k_skinny_expert) when every
-    // matrix is MXFP4; the int8 down or shared expert keeps two kernels
+    const bool skinny = pm == 4 || pm == 5 || (pm == 0 && (size_t)n <= skinny_rows && !many_sh8);
+    // skinny tiles in one kernel per tile (k_skinny_expert); an int8 routed
+    // down keeps two kernels
     const bool fused = skinny && pm != 4 && fusable;
     const int tn = skinny ? kSkTok : kGdTok;
     // a q8_0-split shared expert's down is VALU-heavy: its rows go in small

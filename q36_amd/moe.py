@@ -392,7 +392,8 @@ class MoELayer:
 
     def set_path(self, mode):
         """0 auto (direct for T <= 16, skinny tiles while T*k <= 8*n_expert --
-        16*n_expert in one kernel per tile when the routed down is MXFP4),
+        16*n_expert in one kernel per tile when the routed down is MXFP4, but
+        fat tiles above 1280 tokens when the shared expert is then Q8_0),
         1 sorted (fat tiles), 2 direct, 4 sorted (skinny tiles, gate/up and
         down as two kernels), 5 sorted (skinny tiles, one kernel per tile;
         layers with an int8 down or shared expert take 4); 3 is refused

@@ -718,6 +718,29 @@ def test_down_tile_sizes(q8_shared_layer, which):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("k,T,path", [(1, 1280, 3), (1, 1281, 0), (3, 1280, 3), (3, 1283, 0), (2, 2048, 0), (1, 4096, 0)])
+def test_many_tokens_of_small_top_k(q8_shared_layer, k, T, path):
+    """A Q8_0 shared expert beside MXFP4 tiles leaves the one-kernel form by its
+    tokens, not only by the routed rows; both against the direct path, with the
+    bars of test_down_tile_sizes."""
+    import torch
+    from q36_amd import moe
+    dw = q8_shared_layer["mx"]
+    g = torch.Generator(device="cuda").manual_seed(T + k)
+    x = torch.randn(T, 2048, device="cuda", generator=g)
+    lg = torch.randn(T, 256, device="cuda", generator=g)
+    shg = torch.randn(T, device="cuda", generator=g)
+    layer = moe.MoELayer(T, top_k=k)
+    y = layer.forward(dw, x, lg, shg, out_dtype=torch.float32)
+    assert layer.last_path == path
+    ref = torch.cat([layer.forward(dw, x[t:t + 16], lg[t:t + 16], shg[t:t + 16], out_dtype=torch.float32)
+                     for t in range(0, T, 16)])
+    torch.cuda.synchronize()
+    err = (y - ref).abs().amax(1) / ref.abs().amax(1)
+    assert err.max() <= 5e-3 and err.median() <= 1e-3, (err.max(), err.median())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("scale", [8.0, 2.0 ** 100])
 @pytest.mark.parametrize("k", [8, 1])
 @pytest.mark.parametrize("which,path", [("mxfp4", 1), ("mxfp4", 4), ("mxfp4", 5), ("mx", 0), ("mx", 1), ("mx", 4),
