@@ -3019,10 +3019,14 @@ struct DirectGateupLds {
 // [512w, 512w+512) per 32 to int8 + fp32 scale into LDS and runs its 16
 // blocks against 16 rows of gate and up (int8 MFMA, each block scaled by
 // both scales); partial sums meet in LDS in wave order as in the MXFP4 body.
-// CH K-pairs of weights at a time, two such chunks in flight: all 8 at once
-// (128 registers) at the smallest batches, where one load latency counts; 2
-// from kDirectSh2 tokens, where those registers cost the routed workgroups of
-// the kernel their occupancy (3 waves per SIMD instead of 4).
+// CH K-pairs of weights at a time, two such chunks in flight.  2: all 8 at once
+// (128 registers) cost the routed workgroups of the kernel their occupancy (3
+// waves per SIMD instead of 4).  8 while that occupancy holds them, up to one
+// and a half workgroups per CU (two of two row tiles), or below kDirectSh2
+// tokens; with at most one per CU, 2 again.  Layer, us with 2 / 8: top_k 8, T = 1 (288 workgroups)
+// 10.55 / 10.38, T = 3 (864) 15.1 / 16.2; top_k 2, T = 1 (96) 9.0 / 9.1, T = 4
+// (384) 10.7 / 10.3, T = 5 (480) 11.1 / 11.6, T = 8 (384) 16.0 / 15.4,
+// T = 10 (480) 17.0 / 16.3, T = 11 (528) 18.7 / 20.0.
 constexpr int kDirectSh2 = 3;
 template <int CH>
 __device__ __forceinline__ void direct_shared_q8(const DirectArgs &A, int t, int i, int ft, DirectGateupLds &L_) {
@@ -3254,12 +3258,15 @@ __global__ __launch_bounds__(256) void k_direct_gateup(DirectArgs A) {
 // matrix is q8_0-split (the routed slots with dn_q8, the shared expert with
 // sh_q8) quantise h per 32 to int8 with an fp32 scale (k_quant_q8b) and run
 // each 32-block as one int8 MFMA scaled by both scales (k_gemm_expert_i8).
-// Q8: 0 no such matrix, 1 the shared expert's only, 2 any.  A wave's int8
+// Q8: 0 no such matrix, 1 the shared expert's only, 2 and 3 any.  A wave's int8
 // tile is 64 registers at once; workgroups are 9 waves, so with the 112
 // registers that took, the kernel ran one per CU.  2 fits in 96 registers (two
 // per CU), 1 takes the shared tile in halves and fits in 72 (three per CU);
 // below kDirectSh2 tokens every workgroup fits at once and the second half's
-// latency shows (1 token 10.2 -> 11.2 us), so 2 serves both.  Layer, us at T =
+// latency shows (1 token 10.2 -> 11.2 us), as does the order of 2 (a block's
+// product only after the block before it is scaled, which keeps its results in
+// 96 registers): 3 has neither (layer of 1 token, Q8_0 shared 10.31 -> 10.21 us,
+// at top_k 2 8.98 -> 8.90).  Layer, us at T =
 // 4 / 8 / 16, with the gate/up's chunks: Q8_0 shared 20.9 / 37.2 / 59.2 -> 18.0
 // / 32.1 / 49.4, int8 routed downs too 24.2 / 43.5 / 74.4 -> 22.8 / 40.0 / 67.7
 // (of that 1.0 / 2.4 / 3.7 and 0.7 / 0.9 / 2.4 from the spills, see ac).
@@ -3347,8 +3354,10 @@ __global__ __launch_bounds__(576, Q8 == 2 ? 5 : Q8 == 1 ? 7 : 1) void k_direct_d
 #pragma unroll
             for (int r = 0; r < 4; r++) c[r] = fmaf(q8_scaled(ci[r], w[r], q8_nwb(w[r])), dh, c[r]);
             // one block per scheduling group, as in direct_shared_q8
-            asm volatile("" : "+v"(c));
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Q8 < 3) {
+                asm volatile("" : "+v"(c));
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if ((kb & 1) && (kb >> 1) + NB < NKP) load_q8((kb >> 1) + NB);
         }
     } else {
@@ -4028,18 +4037,22 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             // routing and twice the loads in flight per workgroup; below
             // that, more workgroups spread a small batch better)
             static_assert(kDirectCachedT >= kDirect2Tiles, "cached loads only in the two-tile kernels");
+            const int wgs = n * (FF / (T >= kDirect2Tiles ? 32 : 16));
+            const bool ch8 = wgs > 256 && (wgs <= (T >= kDirect2Tiles ? 512 : 384) || T < kDirectSh2);   // see direct_shared_q8
             if (T >= kDirectCachedT) {
                 if (P.di.sh_q8)
                     hipLaunchKernelGGL((k_direct_gateup<2, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
                 else
                     hipLaunchKernelGGL((k_direct_gateup<0, 2, true>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
             } else if (T >= kDirect2Tiles) {
-                if (P.di.sh_q8)
+                if (P.di.sh_q8 && ch8)
+                    hipLaunchKernelGGL((k_direct_gateup<8, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
+                else if (P.di.sh_q8)
                     hipLaunchKernelGGL((k_direct_gateup<2, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
                 else
                     hipLaunchKernelGGL((k_direct_gateup<0, 2>), dim3(n, FF / 32), dim3(256), 0, s, P.di);
             } else {
-                if (P.di.sh_q8 && T >= kDirectSh2)
+                if (P.di.sh_q8 && !ch8)
                     hipLaunchKernelGGL((k_direct_gateup<2, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
                 else if (P.di.sh_q8)
                     hipLaunchKernelGGL((k_direct_gateup<8, 1>), dim3(n, FF / 16), dim3(256), 0, s, P.di);
@@ -4050,7 +4063,7 @@ static void launch_stage(const Scratch &c, const Plan &P, int st, hipStream_t s)
             const int q8 = P.di.dn_q8 ? 2 : P.di.sh_q8 ? 1 : 0;
             const bool cached = T >= kDirectCachedT;
             const dim3 g(D / 16, T), b(64 * (K + P.has_sh));
-            if (q8 && T < kDirectSh2) hipLaunchKernelGGL((k_direct_down<2, false>), g, b, 0, s, P.di);
+            if (q8 && T < kDirectSh2) hipLaunchKernelGGL((k_direct_down<3, false>), g, b, 0, s, P.di);
             else if (q8 == 2 && cached) hipLaunchKernelGGL((k_direct_down<2, true>), g, b, 0, s, P.di);
             else if (q8 == 2) hipLaunchKernelGGL((k_direct_down<2, false>), g, b, 0, s, P.di);
             else if (q8 && cached) hipLaunchKernelGGL((k_direct_down<1, true>), g, b, 0, s, P.di);

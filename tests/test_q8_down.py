@@ -718,6 +718,28 @@ def test_down_tile_sizes(q8_shared_layer, which):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["mx", "both"])
+@pytest.mark.parametrize("k,T", [(8, 2), (8, 3), (2, 2), (2, 3), (2, 4), (2, 5), (2, 8), (2, 11), (1, 4), (1, 7), (1, 11),
+                                 (1, 12)])
+def test_direct_forms_same_bits(q8_shared_layer, which, k, T):
+    """The forms of the direct kernels (weights in chunks or all at once, one or
+    two row tiles, the down in halves, blocks in order or not) form the same
+    sums: a batch equals its tokens one by one."""
+    import torch
+    from q36_amd import moe
+    g = torch.Generator(device="cuda").manual_seed(10 * T + k)
+    x = torch.randn(T, 2048, device="cuda", generator=g)
+    lg = torch.randn(T, 256, device="cuda", generator=g)
+    shg = torch.randn(T, device="cuda", generator=g)
+    layer = moe.MoELayer(T, top_k=k)
+    y = layer.forward(q8_shared_layer[which], x, lg, shg, out_dtype=torch.float32)
+    one = torch.cat([layer.forward(q8_shared_layer[which], x[t:t + 1], lg[t:t + 1], shg[t:t + 1], out_dtype=torch.float32)
+                     for t in range(T)])
+    torch.cuda.synchronize()
+    assert layer.last_path == 1 and torch.isfinite(y).all() and torch.equal(y, one)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("k,T,path", [(1, 1280, 3), (1, 1281, 0), (3, 1280, 3), (3, 1283, 0), (2, 2048, 0), (1, 4096, 0)])
 def test_many_tokens_of_small_top_k(q8_shared_layer, k, T, path):
     """A Q8_0 shared expert beside MXFP4 tiles leaves the one-kernel form by its
