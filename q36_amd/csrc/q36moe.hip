@@ -2046,8 +2046,8 @@ __device__ __forceinline__ uint2 dn16_pack(float v0, float v1, float v2, float v
 // eb = 15, would be 0 * inf.  A normal c of a group that this raises is still
 // stored at 2 or above, with all of f16's bits.
 __device__ __forceinline__ float dn16_scale(float a, float w, uint32_t &eb) {
-    const uint32_t ew = (__float_as_uint(w) >> 23) & 0xffu;
-    eb = max((__float_as_uint(a) >> 23) & 0xffu, max(ew, 128u) - 113u);
+    const int ew = (__float_as_uint(w) >> 23) & 0xffu;
+    eb = (uint32_t)max(max((int)((__float_as_uint(a) >> 23) & 0xffu), ew - 113), 15);
     return w * __uint_as_float((268u - eb) << 23);
 }
 
