@@ -132,15 +132,26 @@ def kernel_bytes(stage, T, U, shared, dn_q8=False, sh_q8=False):
         dn = U * (Q8_MAT_BYTES if dn_q8 else MAT_BYTES) + (sh_mat if shared else 0)
         return dn + hq, staged
     if stage == "expert":
-        # one kernel per skinny tile: h stays in LDS (the tap copy is written)
+        # one kernel per skinny tile: h stays in LDS (the tap copy is
+        # written); a q8_0-split shared expert has its gate/up here and its
+        # down in the combine
+        if sh_q8:
+            return U * 3 * MAT_BYTES + 2 * sh_mat + xq, hq + T * K * (D * 2 + D // 16)
         return U * 3 * MAT_BYTES + (3 * sh_mat if shared else 0) + xq, hq + staged
+    if stage == "combine":
+        # with the shared down: its matrix, the shared rows of h and the bf16
+        # output; the routed rows' staging read back, the shared rows' written
+        return sh_mat + T * FF + T * FF // 8 + T * D * 2, staged
     raise ValueError(stage)
 
 
-def kernels_of(path):
+def kernels_of(path, sh_q8=False):
     """The grouped-GEMM kernels of a path: one per skinny tile on the
-    one-kernel skinny path (3), else gate/up and down."""
-    return ("expert",) if path == 3 else ("gateup", "down")
+    one-kernel skinny path (3), with the combine where that holds the shared
+    down (a q8_0-split shared expert), else gate/up and down."""
+    if path == 3:
+        return ("expert", "combine") if sh_q8 else ("expert",)
+    return "gateup", "down"
 
 
 def kernel_us(st_us, kernel):
@@ -149,9 +160,14 @@ def kernel_us(st_us, kernel):
     return st_us["gateup"] if kernel == "expert" else st_us[kernel]
 
 
-def kernel_flops(stage, T, shared):
+def kernel_flops(stage, T, shared, sh_q8=False):
+    gu, dn = 2 * D * 2 * FF, 2 * FF * D
     P = T * K + (T if shared else 0)
-    return P * {"gateup": 2 * D * 2 * FF, "down": 2 * FF * D, "expert": 3 * 2 * FF * D}[stage]
+    if stage == "expert":
+        return P * (gu + dn) - (T * dn if sh_q8 else 0)
+    if stage == "combine":      # the shared down of a q8_0-split shared expert
+        return T * dn
+    return P * {"gateup": gu, "down": dn}[stage]
 
 
 def measured_traffic(config, stage):
@@ -365,9 +381,9 @@ class Bench:
              "layer_bytes": by, "layer_hbm_frac": by / (ms_layer * 1e-3) / 1e9 / HBM_PEAK_GBS,
              "layer_flops": fl, "layer_mfma_frac": fl / (ms_layer * 1e-3) / 1e12 / MFMA_FP8_PEAK_TFS,
              "stage_us": st_us}
-        for st in kernels_of(path):
+        for st in kernels_of(path, sh_q8):
             us = kernel_us(st_us, st)
-            kf = kernel_flops(st, T, shared)
+            kf = kernel_flops(st, T, shared, sh_q8)
             kb, ko = kernel_bytes(st, T, U, shared, dn_q8, sh_q8)
             r[st] = {"us": us, "mfma_frac": kf / (us * 1e-6) / 1e12 / MFMA_FP8_PEAK_TFS,
                      "hbm_frac": kb / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, "flops": kf, "bytes": kb,
@@ -470,10 +486,10 @@ def main():
 
     U, path, st_us = B.stage_times()
     head = B.summary(ms, U, path, st_us, dn_q8, sh_q8)
-    dom = max(kernels_of(path), key=lambda k: kernel_us(st_us, k))
+    dom = max(kernels_of(path, sh_q8), key=lambda k: kernel_us(st_us, k))
     prefill = T >= 256
     if prefill:
-        fl = kernel_flops(dom, T, shared)
+        fl = kernel_flops(dom, T, shared, sh_q8)
         ach = fl / (kernel_us(st_us, dom) * 1e-6) / 1e12
         roof = {"bound": "mfma", "achieved": ach, "peak": MFMA_FP8_PEAK_TFS, "unit": "TFLOP/s",
                 "frac": ach / MFMA_FP8_PEAK_TFS, "traffic": None, "kernel": dom,
@@ -518,7 +534,7 @@ def main():
         "distinct_experts": U,
         "stage_us": st_us,
         "roofline": roof,
-        "grouped_gemms": {st: head[st] for st in kernels_of(path)},
+        "grouped_gemms": {st: head[st] for st in kernels_of(path, sh_q8)},
     }
     # the other BASELINE configurations, measured in the same run on the same
     # weight layers: a HIP graph of one forward per layer, median of replays

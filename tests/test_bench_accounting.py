@@ -23,6 +23,22 @@ def test_decode1_bytes():
     assert flops == 8 * 6_291_456
 
 
+def test_shared_down_in_the_combine():
+    # a Q8_0 shared expert of a small batch: its gate/up with the tiles, its
+    # down with the combine; together what gate/up and down count
+    q8 = bench.Q8_MAT_BYTES
+    assert bench.kernels_of(3, True) == ("expert", "combine") and bench.kernels_of(3) == ("expert",)
+    alg, ovh = bench.kernel_bytes("expert", 40, 180, True, sh_q8=True)
+    assert alg == 180 * 1_671_168 + 2 * q8 + 40 * (2048 + 64) + 40 * (2048 + 256)
+    assert ovh == 320 * (512 + 16) + 40 * (512 + 64) + 320 * (2048 * 2 + 128)
+    alg, ovh = bench.kernel_bytes("combine", 40, 180, True, sh_q8=True)
+    assert alg == q8 + 40 * (512 + 64) + 40 * 4096
+    assert ovh == 360 * (2048 * 2 + 128)
+    assert (bench.kernel_flops("expert", 40, True, True) + bench.kernel_flops("combine", 40, True, True)
+            == bench.kernel_flops("gateup", 40, True) + bench.kernel_flops("down", 40, True)
+            == bench.kernel_flops("expert", 40, True))
+
+
 def test_prefill_down_is_weights_plus_h():
     # 142.6 MB of weights + 17.3 MB of h; the staging is overhead
     alg, ovh = bench.kernel_bytes("down", 4096, 256, False)
