@@ -814,11 +814,11 @@ __device__ __forceinline__ void wave_scan256(const int *v, int n, int *out, int 
 // Up to kScanInlineBlocks routing blocks (8192 tokens) each workgroup also
 // does the column scan itself (inline_cols) and k_colscan is not launched:
 // the counts are a byte each, 256 per block, so one 16-byte load per lane
-// covers 16 blocks over the workgroup, and all of a lane's loads are in
-// flight together.  A count is at most 16, so the sums over up to 512 blocks
-// fit the bytes' 16-bit widenings.  Beyond, the workgroups' reads grow with
-// the square of the tokens, and the separate scan, which reads each count
-// once, takes over.  us of the scan stage, against a count per int in
+// covers 16 blocks over the workgroup, and a lane's loads of 256 blocks are in
+// flight together (T > 4096: two such rounds).  A count is at most 16, so the
+// sums over up to 512 blocks fit the bytes' 16-bit widenings.  Beyond, the
+// workgroups' reads grow with the square of the tokens, and the separate scan,
+// which reads each count once, takes over.  us of the scan stage, against a count per int in
 // expert-major order, scanned by each workgroup up to 64 blocks and by
 // k_colscan above:
 //   T = 1000     17.0 -> 5.8            T = 4096   5.1 + 6.0 -> 7.9
@@ -1580,8 +1580,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // wave walks the tokens with its row in registers (from some 3000 rows on, when
 // enough waves share a CU to cover a load, without PIN: 16 tokens and 1025 /
 // 2049 / 4097 rows 8.6 / 10.4 / 21.0 us with it, 10.1 / 11.3 / 18.7 without).
-// Same products and order of sums whatever T.  us at T = 1 / 4 / 7 / 9 / 16, one wave per row against the
-// waves per token (launch_router's limits):
+// Same products and order of sums whatever T.  us at T = 1 / 4 / 7 / 9 / 16, one
+// wave per row against the waves per token (launch_router's limits):
 //    257 rows   2.4 / 3.5 / 5.0 /  5.4 /  8.1    2.4 / 2.7 / 3.5 /  4.6 /  4.7
 //    513        2.5 / 3.6 / 5.1 /  5.5 /  8.3    2.5 / 3.1 / 4.3 /  5.9 /  6.1
 //    769        2.5 / 3.7 / 5.2 /  5.6 /  8.4    2.5 / 3.5 / 5.2 /  7.2 /  7.5

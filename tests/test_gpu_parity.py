@@ -825,12 +825,17 @@ def test_scan_order(dev, T, E):
 
 # every tile shape of the fp16 router at its edges: 257 rows (the last row
 # block takes a fifth tile) and row counts around a block, T at both sides of
-# each rule and with remainders
+# each rule and with remainders.  In order: 1x1 and 2x2; 2x4 and 4x4 with the
+# fifth tile; 4x4 without; few rows in 2x2 and 1x1; 2x4 and 4x4 with the fifth
+# tile and f32 x; 4x4 of one block (65, 80 rows: 5 tiles) and of two (81), 2x4
+# of one.  Each shape in either x format.
 @pytest.mark.parametrize("T,n_expert,n_rows,bf16", [
     (17, 256, 257, False), (17, 256, 257, True), (337, 256, 257, False), (361, 256, 257, True),
     (1567, 256, 257, False), (1601, 256, 257, True), (2048, 256, 257, False), (2049, 256, 257, True),
     (2113, 256, 256, False), (4097, 80, 81, False), (4099, 80, 80, True), (9001, 1, 2, False), (70, 63, 64, False),
-    (12001, 16, 17, True)])
+    (12001, 16, 17, True),
+    (1601, 256, 257, False), (2049, 256, 257, False), (4099, 256, 257, False), (8209, 64, 65, False), (8193, 79, 80, True),
+    (4805, 80, 81, False), (4833, 80, 81, True), (8192, 64, 65, False)])
 def test_router_f16_tiles(dev, T, n_expert, n_rows, bf16):
     rng = np.random.default_rng(700 + T)
     w = (rng.standard_normal((n_rows, 2048)) * 0.02).astype(np.float32)

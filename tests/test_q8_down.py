@@ -687,7 +687,9 @@ def test_q8_shared_taps_and_replays(q8_shared_layer, T):
 def test_down_tile_sizes(q8_shared_layer, which):
     """Fat tiles whose row counts sit on the edges of the down kernels' chunks
     and column tiles (int8 and MXFP4 routed downs, with and without the int8
-    shared tiles beside them) against the direct path, which has no tiles."""
+    shared tiles beside them) against the direct path, which has no tiles: the
+    edges of chunks and tiles, not the accuracy, for which test_forward_q8_shared
+    and test_forward_q8_down compare with the oracle."""
     import torch
     from q36_amd import moe
     dw = q8_shared_layer[which.split(",")[0]]
