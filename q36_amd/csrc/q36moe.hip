@@ -1573,21 +1573,30 @@ __device__ __forceinline__ float wave_sum(float v) {
 // Workgroup = one router row.  With few rows a wave takes NT tokens (w,
 // w + waves, ...), so the tokens' dot products run side by side where one wave
 // walking the tokens pays an L2 round trip for each: up to kRfW tokens a wave
-// per token (NW = 0: no loop and no count of waves to read), beyond that NW =
-// kRfW waves of two tokens, so that a wave's row and tokens are all in flight
-// at once (16 waves leave 64 registers each, which a row and a token fill).
-// With many rows, whose waves fill the chip and share the L1's bandwidth, one
-// wave walks the tokens with its row in registers (from some 3000 rows on, when
-// enough waves share a CU to cover a load, without PIN: 16 tokens and 1025 /
-// 2049 / 4097 rows 8.6 / 10.4 / 21.0 us with it, 10.1 / 11.3 / 18.7 without).
-// Same products and order of sums whatever T.  us at T = 1 / 4 / 7 / 9 / 16, one
-// wave per row against the waves per token (launch_router's limits):
-//    257 rows   2.4 / 3.5 / 5.0 /  5.4 /  8.1    2.4 / 2.7 / 3.5 /  4.6 /  4.7
-//    513        2.5 / 3.6 / 5.1 /  5.5 /  8.3    2.5 / 3.1 / 4.3 /  5.9 /  6.1
-//    769        2.5 / 3.7 / 5.2 /  5.6 /  8.4    2.5 / 3.5 / 5.2 /  7.2 /  7.5
-//   1025        2.6 / 3.9 / 5.4 /  5.8 /  8.6    2.6 / 3.9 / 6.1 /  8.5 /  8.8
-//   4097        4.2 / 7.3 /11.7 / 12.8 / 21      4.2 / 9.8 /17.3 / 25   / 26.5
-constexpr int kRfW = 8;
+// per token (NW = 0: no loop and no count of waves to read), beyond that
+// kRfL waves of two tokens, or kRfW where the rows leave CUs idle (up to 192)
+// or the tokens fill their rounds (from 256), which leaves a wave registers for
+// its row and both tokens.  With many rows, whose waves fill the chip and share the L1's
+// bandwidth, one wave walks the tokens with its row in registers (fp32 x and
+// more than 2560 rows, when enough waves share a CU to cover a load, without
+// PIN: 16 tokens and 2049 / 3073 / 4097 rows 11.2 / 16.1 / 22.1 us with it,
+// 12.1 / 15.2 / 19.9 without; bf16 x the same either way).  Over hundreds of
+// tokens (with bf16 x, whose conversions take issue slots, over dozens past
+// 2560 rows) the walk's chain of round trips counts again.
+// Same products and order of sums whatever T.  us, fp32 x, one wave walking
+// against the waves per token (T <= 8) or kRfL waves of two (beyond):
+//    rows  T = 4         8           9           16          64          512
+//     257  4.4 /  3.7   5.9 /  4.4   6.3 /  4.8   9.0 /  5.4    28 / 12   272 /  68
+//     769  4.6 /  4.5   6.1 /  6.3   6.5 /  6.3   9.3 /  7.8    28 / 20   278 / 131
+//    1025  4.8 /  4.9   6.3 /  7.2   6.6 /  7.2   9.4 /  9.0    29 / 24   279 / 171
+//    1537  4.9 /  5.8   6.6 /  8.8   7.0 /  8.9   9.8 / 11.1    30 / 31   280 / 222
+//    2049  5.5 /  6.7   7.3 / 10.7   7.7 / 10.2  11.2 / 13.4    35 / 40   279 / 291
+//    4097  8.0 / 10.8  11.8 / 18.0  12.8 / 17.5  19.9 / 23.7    68 / 73   493 / 538
+// (bf16 x: 2049 rows, 512 tokens 302 / 270, 4097 rows, 64 / 512 tokens 76 / 69,
+// 592 / 499.)  kRfW against kRfL waves of two tokens, 9 tokens: 257 / 769 rows 5.5
+// / 8.3 against 4.8 / 6.3; 16: 129 rows 4.6 against 4.9; 512: 129 / 257 / 1025
+// rows 41 / 66 / 166 against 66 / 68 / 171.
+constexpr int kRfW = 8, kRfL = 4;
 template <int XF, int NT, int NW, bool PIN = true>
 __global__ __launch_bounds__(64 * (NW ? NW : kRfW)) void k_router_f32(const float *__restrict__ W, int n_expert,
                                                                      const void *__restrict__ x, int T,
@@ -1827,12 +1836,18 @@ static void launch_router(bool f16, const float *w, int n_rows, int n_expert, co
     if (!f16) {
         if (T == 1 || (T <= kRfW && n_rows <= 768))
             hipLaunchKernelGGL((k_router_f32<XF, 1, 0>), dim3(n_rows), dim3(64 * T), 0, s, w, n_expert, x, T, logits, ld, shg);
-        else if (T > kRfW && n_rows <= 512)
-            hipLaunchKernelGGL((k_router_f32<XF, 2, kRfW>), dim3(n_rows), dim3(64 * kRfW), 0, s, w, n_expert, x, T, logits, ld,
-                               shg);
-        else if (n_rows <= 3072)
+        else if (T > kRfW && (n_rows <= 768 || (n_rows <= 1152 && T >= 16) || (n_rows <= 2560 && T >= 256) ||
+                              (XF == Q36MOE_FMT_BF16 && n_rows > 2560 && T >= 32))) {
+            if (n_rows <= 192 || T >= 256)
+                hipLaunchKernelGGL((k_router_f32<XF, 2, kRfW>), dim3(n_rows), dim3(64 * kRfW), 0, s, w, n_expert, x, T, logits,
+                                   ld, shg);
+            else
+                hipLaunchKernelGGL((k_router_f32<XF, 2, kRfL>), dim3(n_rows), dim3(64 * kRfL), 0, s, w, n_expert, x, T, logits,
+                                   ld, shg);
+        }
+        else if (XF == Q36MOE_FMT_BF16 || n_rows <= 2560)
             hipLaunchKernelGGL((k_router_f32<XF, 1, 1>), dim3(n_rows), dim3(64), 0, s, w, n_expert, x, T, logits, ld, shg);
-        else
+        else if constexpr (XF == Q36MOE_FMT_F32)
             hipLaunchKernelGGL((k_router_f32<XF, 1, 1, false>), dim3(n_rows), dim3(64), 0, s, w, n_expert, x, T, logits, ld,
                                shg);
         return;

@@ -859,19 +859,24 @@ def test_router_f16_tiles(dev, T, n_expert, n_rows, bf16):
 
 
 @pytest.mark.parametrize("T,n_rows", [(1, 257), (2, 257), (8, 257), (9, 257), (15, 257), (16, 257), (17, 257), (35, 257),
-                                      (1, 769), (8, 768), (8, 769), (9, 512), (9, 513), (33, 513), (9, 3072), (5, 3073)])
-def test_router_f32_waves(dev, T, n_rows):
-    """A wave per token up to 8 tokens, eight waves of two tokens in a loop
-    beyond, one wave walking the tokens where there are many rows: the same
+                                      (1, 769), (8, 768), (8, 769), (9, 512), (9, 513), (33, 513), (9, 3072), (5, 3073),
+                                      (9, 768), (9, 769), (15, 1152), (16, 1152), (16, 1153), (255, 2560), (261, 2560),
+                                      (256, 2561), (13, 192), (13, 193), (255, 257), (259, 257)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_router_f32_waves(dev, T, n_rows, bf16):
+    """A wave per token up to 8 tokens, four or eight waves of two tokens in a
+    loop beyond, one wave walking the tokens where there are many rows: the same
     sums as the tokens one by one."""
     rng = np.random.default_rng(800 + T)
     w = torch.from_numpy((rng.standard_normal((n_rows, 2048)) * 0.02).astype(np.float32)).to(dev)
     x = torch.from_numpy(rng.standard_normal((T, 2048), dtype=np.float32)).to(dev)
+    if bf16:
+        x = x.to(torch.bfloat16)
     lg, shg = moe.router_logits(w, x, n_rows - 1, moe.ROUTER_F32)
     one = [moe.router_logits(w, x[t:t + 1].contiguous(), n_rows - 1, moe.ROUTER_F32) for t in range(T)]
     torch.cuda.synchronize()
     assert torch.equal(lg, torch.cat([o[0] for o in one])) and torch.equal(shg, torch.cat([o[1] for o in one]))
-    ref, mag = _router_ref(w.cpu().numpy(), x.cpu().numpy(), False)
+    ref, mag = _router_ref(w.cpu().numpy(), x.float().cpu().numpy(), False)
     got = torch.cat([lg, shg[:, None]], 1).cpu().numpy().astype(np.float64)
     assert (np.abs(got - ref) / mag).max() <= 2e-6
 
